@@ -4,8 +4,8 @@
  * Every entry point takes device pointers the caller owns, sizes and element
  * strides by value, and an optional HIP stream (`void*` = hipStream_t, NULL =
  * the null stream).  Nothing here allocates, copies or synchronises: a call
- * validates its arguments on the host, enqueues one kernel on `stream` and
- * returns.  Validation happens before any HIP call, so argument errors are
+ * validates its arguments on the host, enqueues one kernel on `stream`
+ * (neso_w8a16_matmul_ws: one or two) and returns.  Validation happens before any HIP call, so argument errors are
  * reported on hosts without a GPU.
  *
  * fp16 buffers are IEEE binary16, passed as `const void*`.
@@ -263,6 +263,22 @@ int neso_w8a16_matmul(const void* A, const int8_t* B, float* C, int32_t K, int32
 int neso_w8a16_scaled_matmul(const void* A, const int8_t* B, float* C, const void* scale,
                              int32_t K, int32_t stride_am, int32_t stride_bk, int32_t stride_cm,
                              int32_t M, int32_t N, void* stream);
+
+/*
+ * The two W8A16 matmuls above (scale NULL: unscaled) with a workspace.  For
+ * few rows of A the chip is only filled when K is split over workgroups,
+ * whose fp32 partial sums meet in `workspace` (device memory the caller
+ * owns, 16-byte aligned, not shared with another launch in flight) and are
+ * added in a fixed order by a second kernel on `stream`.
+ * neso_w8a16_workspace_bytes gives the size that such a call uses on the
+ * current device, 0 if it uses none; a smaller workspace, or NULL, runs
+ * the call without the split.
+ */
+int64_t neso_w8a16_workspace_bytes(const void* A, const int8_t* B, int32_t K, int32_t stride_am,
+                                   int32_t stride_bk, int32_t M, int32_t N);
+int neso_w8a16_matmul_ws(const void* A, const int8_t* B, float* C, const void* scale, int32_t K,
+                         int32_t stride_am, int32_t stride_bk, int32_t stride_cm, int32_t M, int32_t N,
+                         void* workspace, int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -1210,12 +1210,32 @@ constexpr char kManifest[] = R"JSON({
    },
    "variants": [
     {
+     "device_kernel": "w8a16_skinny_kernel",
+     "source": "neso_amd/csrc/qmatmul_w8_skinny.hip",
+     "template_params": [
+      "MT"
+     ],
+     "when": "M <= 64 under w8a16_gemm_kernel's alignment: 128-column strips; with a workspace (neso_w8a16_matmul_ws) K is split over min(cus // strips, K // 256, 8) workgroups per strip and w8a16_reduce_kernel follows",
+     "threadgroup_size": "256",
+     "num_warps": "4",
+     "grid": [
+      "cdiv(N, 128)",
+      "1",
+      "1"
+     ],
+     "constants": {
+      "block_m": "16 * MT",
+      "block_n": "128",
+      "block_k": "32"
+     }
+    },
+    {
      "device_kernel": "w8a16_gemm_kernel",
      "source": "neso_amd/csrc/qmatmul.hip",
      "template_params": [
       "T"
      ],
-     "when": "K, N, lda, ldb multiples of 8 and A 16-byte / B 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64)",
+     "when": "M > 64, K, N, lda, ldb multiples of 8 and A 16-byte / B 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64)",
      "threadgroup_size": "2 * T",
      "num_warps": "T // 32",
      "grid": [
@@ -1335,12 +1355,32 @@ constexpr char kManifest[] = R"JSON({
    },
    "variants": [
     {
+     "device_kernel": "w8a16_skinny_kernel",
+     "source": "neso_amd/csrc/qmatmul_w8_skinny.hip",
+     "template_params": [
+      "MT"
+     ],
+     "when": "M <= 64 under w8a16_gemm_kernel's alignment: 128-column strips; with a workspace (neso_w8a16_matmul_ws) K is split over min(cus // strips, K // 256, 8) workgroups per strip and w8a16_reduce_kernel follows",
+     "threadgroup_size": "256",
+     "num_warps": "4",
+     "grid": [
+      "cdiv(N, 128)",
+      "1",
+      "1"
+     ],
+     "constants": {
+      "block_m": "16 * MT",
+      "block_n": "128",
+      "block_k": "32"
+     }
+    },
+    {
      "device_kernel": "w8a16_gemm_kernel",
      "source": "neso_amd/csrc/qmatmul.hip",
      "template_params": [
       "T"
      ],
-     "when": "K, N, lda, ldb multiples of 8 and A 16-byte / B 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64)",
+     "when": "M > 64, K, N, lda, ldb multiples of 8 and A 16-byte / B 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64)",
      "threadgroup_size": "2 * T",
      "num_warps": "T // 32",
      "grid": [

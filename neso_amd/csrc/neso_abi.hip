@@ -502,9 +502,11 @@ int neso_w4a16_matmul(const void* X, const int32_t* W, const void* scales, void*
   return launched(neso::launch_w4a16(a, static_cast<hipStream_t>(stream)), name);
 }
 
-static int w8a16_common(const void* A, const int8_t* B, float* C, const void* scale, int32_t K,
-                        int32_t stride_am, int32_t stride_bk, int32_t stride_cm, int32_t M,
-                        int32_t N, void* stream, const char* name) {
+// Fills `a` for a checked, non-empty call; *empty is set for a no-op.
+static int w8a16_args(neso::W8Args& a, bool* empty, const void* A, const int8_t* B, float* C,
+                      const void* scale, int32_t K, int32_t stride_am, int32_t stride_bk,
+                      int32_t stride_cm, int32_t M, int32_t N, const char* name) {
+  *empty = true;
   if (!A || !B || !C) return fail(NESO_EINVAL, "%s: null tensor pointer", name);
   if (M < 0 || N < 0 || K < 0) return fail(NESO_EINVAL, "%s: negative size", name);
   if (stride_am < K || stride_bk < N || stride_cm < N)
@@ -518,7 +520,6 @@ static int w8a16_common(const void* A, const int8_t* B, float* C, const void* sc
       !extent32((int64_t)(K - 1) * stride_bk + N))
     return fail(NESO_EINVAL, "%s: A or B spans 4 GiB or more (M=%d, K=%d, stride_am=%d, "
                 "stride_bk=%d)", name, M, K, stride_am, stride_bk);
-  neso::W8Args a{};
   a.A = static_cast<const neso::half_t*>(A);
   a.B = B;
   a.C = C;
@@ -529,12 +530,24 @@ static int w8a16_common(const void* A, const int8_t* B, float* C, const void* sc
   a.lda = stride_am;
   a.ldb = stride_bk;
   a.ldc = stride_cm;
-  return launched(neso::launch_w8a16(a, static_cast<hipStream_t>(stream)), name);
+  *empty = false;
+  return ok();
+}
+
+static int w8a16_common(const void* A, const int8_t* B, float* C, const void* scale, int32_t K,
+                        int32_t stride_am, int32_t stride_bk, int32_t stride_cm, int32_t M,
+                        int32_t N, void* workspace, int64_t workspace_bytes, void* stream,
+                        const char* name) {
+  neso::W8Args a{};
+  bool empty;
+  const int st = w8a16_args(a, &empty, A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N, name);
+  if (st != NESO_OK || empty) return st;
+  return launched(neso::launch_w8a16(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream)), name);
 }
 
 int neso_w8a16_matmul(const void* A, const int8_t* B, float* C, int32_t K, int32_t stride_am,
                       int32_t stride_bk, int32_t stride_cm, int32_t M, int32_t N, void* stream) {
-  return w8a16_common(A, B, C, nullptr, K, stride_am, stride_bk, stride_cm, M, N, stream,
+  return w8a16_common(A, B, C, nullptr, K, stride_am, stride_bk, stride_cm, M, N, nullptr, 0, stream,
                       "w8a16_matmul");
 }
 
@@ -542,8 +555,29 @@ int neso_w8a16_scaled_matmul(const void* A, const int8_t* B, float* C, const voi
                              int32_t K, int32_t stride_am, int32_t stride_bk, int32_t stride_cm,
                              int32_t M, int32_t N, void* stream) {
   if (!scale) return fail(NESO_EINVAL, "w8a16_scaled_matmul: null scale pointer");
-  return w8a16_common(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N, stream,
+  return w8a16_common(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N, nullptr, 0, stream,
                       "w8a16_scaled_matmul");
+}
+
+int64_t neso_w8a16_workspace_bytes(const void* A, const int8_t* B, int32_t K, int32_t stride_am,
+                                   int32_t stride_bk, int32_t M, int32_t N) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  neso::W8Args a{};
+  a.A = static_cast<const neso::half_t*>(A);
+  a.B = B;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.lda = stride_am;
+  a.ldb = stride_bk;
+  return neso::w8a16_workspace_bytes(a);
+}
+
+int neso_w8a16_matmul_ws(const void* A, const int8_t* B, float* C, const void* scale, int32_t K,
+                         int32_t stride_am, int32_t stride_bk, int32_t stride_cm, int32_t M, int32_t N,
+                         void* workspace, int64_t workspace_bytes, void* stream) {
+  return w8a16_common(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N, workspace, workspace_bytes,
+                      stream, scale ? "w8a16_scaled_matmul" : "w8a16_matmul");
 }
 
 }  // extern "C"

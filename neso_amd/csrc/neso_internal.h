@@ -129,7 +129,17 @@ struct W8Args {
   int32_t lda, ldb, ldc;
 };
 
-hipError_t launch_w8a16(const W8Args& a, hipStream_t stream);
+// Few rows of A (qmatmul_w8_skinny.hip), under w8a16_tiled's conditions:
+// M <= w8a16_skinny_max_m().  `splits` > 1 (at most w8a16_skinny_splits())
+// splits K over workgroups and needs a workspace of splits * M * N floats,
+// 16-byte aligned.
+int w8a16_skinny_max_m();
+int w8a16_skinny_splits(const W8Args& a);
+hipError_t launch_w8a16_skinny(const W8Args& a, int splits, float* workspace, hipStream_t stream);
+
+// The workspace launch_w8a16 can use for this call, in bytes (0: none).
+int64_t w8a16_workspace_bytes(const W8Args& a);
+hipError_t launch_w8a16(const W8Args& a, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
 // Rel-pos bias precompute: Q_u = Q + bias_u and the unscaled dense
 // rel_bias[h][i][j] = (Q + bias_v)[h][i] . K_rel[h][T-1-i+j], fp32 in, fp16

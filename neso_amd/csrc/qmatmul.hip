@@ -1328,16 +1328,32 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   return launch<&w4a16_mfma_kernel<TN>>(ktag("w4a16_mfma_kernel", TN), grid, dim3(kThreads), s, a);
 }
 
-hipError_t launch_w8a16(const W8Args& a, hipStream_t s) {
-  // The tiled kernel reads A and B in 16-byte pieces: A's must be 16-byte
-  // aligned and never straddle the end of a row; B's need 8-byte alignment
-  // (a piece that straddles N reads columns that are never stored).  Buffer
-  // offsets stay below 2^31 bytes.
-  const bool tiled = a.K % 8 == 0 && a.lda % 8 == 0 && a.N % 8 == 0 && a.ldb % 8 == 0 &&
-                     (reinterpret_cast<uintptr_t>(a.A) & 15u) == 0 &&
-                     (reinterpret_cast<uintptr_t>(a.B) & 7u) == 0 &&
-                     (int64_t)256 * a.lda * 2 < ((int64_t)1 << 31) &&
-                     (int64_t)a.K * a.ldb < ((int64_t)1 << 31);
+// The tiled and skinny kernels read A and B in 16- and 8-byte pieces: A's
+// must be 16-byte aligned and never straddle the end of a row; B's need
+// 8-byte alignment (a 16-byte piece that straddles N reads columns that are
+// never stored).  Buffer offsets stay below 2^31 bytes.
+static bool w8a16_tiled(const W8Args& a) {
+  return a.K % 8 == 0 && a.lda % 8 == 0 && a.N % 8 == 0 && a.ldb % 8 == 0 &&
+         (reinterpret_cast<uintptr_t>(a.A) & 15u) == 0 &&
+         (reinterpret_cast<uintptr_t>(a.B) & 7u) == 0 &&
+         (int64_t)256 * a.lda * 2 < ((int64_t)1 << 31) &&
+         (int64_t)a.K * a.ldb < ((int64_t)1 << 31);
+}
+
+int64_t w8a16_workspace_bytes(const W8Args& a) {
+  if (a.M > w8a16_skinny_max_m() || !w8a16_tiled(a)) return 0;
+  const int splits = w8a16_skinny_splits(a);
+  return splits > 1 ? (int64_t)splits * a.M * a.N * 4 : 0;
+}
+
+hipError_t launch_w8a16(const W8Args& a, void* workspace, int64_t workspace_bytes, hipStream_t s) {
+  const bool tiled = w8a16_tiled(a);
+  if (tiled && a.M <= w8a16_skinny_max_m()) {
+    const int64_t need = w8a16_workspace_bytes(a);
+    const bool split = need && workspace && workspace_bytes >= need &&
+                       (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
+    return launch_w8a16_skinny(a, split ? w8a16_skinny_splits(a) : 1, static_cast<float*>(workspace), s);
+  }
   if (tiled) {
     // 256 x 256 tiles (a third fewer LDS bytes per MFMA) when they still
     // give every CU a workgroup; 128 x 128 otherwise.

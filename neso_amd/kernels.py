@@ -428,27 +428,45 @@ def _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N) -> Non
         _extent(scale, "scale", N)
 
 
+def _w8(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N, stream) -> None:
+    _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N)
+    lib = _lib.load()
+    M, N, K = int(M), int(N), int(K)
+    stride_am, stride_bk, stride_cm = int(stride_am), int(stride_bk), int(stride_cm)
+    a, b = _ptr(A, "A", torch.float16), _ptr(B, "B", torch.int8)
+    c = _ptr(C, "C", torch.float32)
+    s = None if scale is None else _ptr(scale, "scale", torch.float16)
+    st = _stream(stream, A, C)
+    # Partial sums of a K split, where the call has one.  The workspace comes
+    # from torch's allocator on the launch stream, so it is reused only in
+    # that stream's order (and stays in the pool of a captured graph).
+    ws = None
+    if isinstance(A, torch.Tensor):
+        need = lib.neso_w8a16_workspace_bytes(a, b, K, stride_am, stride_bk, M, N)
+        if need:
+            with _on_stream(st, A.device), contextlib.suppress(torch.cuda.OutOfMemoryError):
+                ws = torch.empty(need // 4, dtype=torch.float32, device=A.device)
+    w, need = (0, 0) if ws is None else (ws.data_ptr(), ws.numel() * 4)
+    if s is None:
+        status = lib.neso_w8a16_matmul_ws(a, b, c, None, K, stride_am, stride_bk, stride_cm, M, N, w, need, st)
+    else:
+        if not s:  # the scaled entry point rejects a null scale
+            status = lib.neso_w8a16_scaled_matmul(a, b, c, s, K, stride_am, stride_bk, stride_cm, M, N, st)
+        else:
+            status = lib.neso_w8a16_matmul_ws(a, b, c, s, K, stride_am, stride_bk, stride_cm, M, N, w, need, st)
+    _lib.check(status)
+
+
 def w8a16_matmul(A, B, C, K: int, stride_am: int, stride_bk: int, stride_cm: int, *, M: int,
                  N: int, stream=None) -> None:
     """C fp32 = A fp16 @ f16(B int8 [K, N]) (tests/test_quantized_matmul.py:77-80 order)."""
-    _w8_extents(A, B, C, None, K, stride_am, stride_bk, stride_cm, M, N)
-    lib = _lib.load()
-    st = lib.neso_w8a16_matmul(
-        _ptr(A, "A", torch.float16), _ptr(B, "B", torch.int8), _ptr(C, "C", torch.float32), int(K),
-        int(stride_am), int(stride_bk), int(stride_cm), int(M), int(N), _stream(stream, A, C))
-    _lib.check(st)
+    _w8(A, B, C, None, K, stride_am, stride_bk, stride_cm, M, N, stream)
 
 
 def w8a16_scaled_matmul(A, B, C, scale, K: int, stride_am: int, stride_bk: int, stride_cm: int,
                         *, M: int, N: int, stream=None) -> None:
     """C = (A @ f16(B)) * scale[n] (tests/test_quantized_matmul.py:189-192 order)."""
-    _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N)
-    lib = _lib.load()
-    st = lib.neso_w8a16_scaled_matmul(
-        _ptr(A, "A", torch.float16), _ptr(B, "B", torch.int8), _ptr(C, "C", torch.float32),
-        _ptr(scale, "scale", torch.float16), int(K), int(stride_am), int(stride_bk),
-        int(stride_cm), int(M), int(N), _stream(stream, A, C))
-    _lib.check(st)
+    _w8(A, B, C, 0 if scale is None else scale, K, stride_am, stride_bk, stride_cm, M, N, stream)
 
 
 KERNELS = {
