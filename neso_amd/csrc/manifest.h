@@ -1008,7 +1008,7 @@ constexpr char kManifest[] = R"JSON({
       "R",
       "PS"
      ],
-     "when": "M <= 2 and K <= 8192: GEMV, one wave per R output rows, MR rows of X",
+     "when": "M <= 2 and K <= 8192, or N >= 1024 and K <= 16384 and (M = 1 or M = 2 and N < 16 cus): GEMV, one wave per R output rows, MR rows of X",
      "threadgroup_size": "256",
      "num_warps": "4",
      "grid": [
@@ -1027,9 +1027,11 @@ constexpr char kManifest[] = R"JSON({
      "template_params": [
       "WV",
       "T",
-      "QWMAX"
+      "QWMAX",
+      "GS",
+      "MP"
      ],
-     "when": "3 <= M <= 16, group 32, K % 128 == 0, K <= 4096: X in LDS, WV waves split K, T 16-column tiles per workgroup",
+     "when": "K % 128 == 0 and a power-of-two group: X in LDS, WV waves split K, T 16-column tiles per workgroup, GS scales per 128 codes; 3 <= M <= 16 (QWMAX = 4): K <= 4096, or any K (MP = 1, phases of at most 4096) with group > 32 or N >= 1024 and (M <= 8 or K <= 8192); 17 <= M <= 32 (QWMAX = 2, phases of at most 2048): K >= 1024, N >= 1024 and 8 K >= N",
      "threadgroup_size": "64 * WV",
      "num_warps": "WV",
      "grid": [

@@ -114,9 +114,11 @@ struct W4Args {
 };
 
 hipError_t launch_w4a16(const W4Args& a, hipStream_t stream);
-// Skinny-M kernel with X in LDS (qmatmul_skinny.hip): M <= 16, group 32,
-// K % 128 == 0, K <= w4a16_skinny_lds_max_k().
+// Skinny-M kernel with X in LDS (qmatmul_skinny.hip): M <= 32 and
+// w4a16_skinny_lds_groups(); M <= 16 rows run in one phase up to K =
+// w4a16_skinny_lds_max_k().
 int w4a16_skinny_lds_max_k();
+bool w4a16_skinny_lds_groups(const W4Args& a);
 hipError_t launch_w4a16_skinny_lds(const W4Args& a, hipStream_t stream);
 
 // C[M][N] (f32) = A[M][K] (f16) * f16(B[K][N] int8) [* scale[n]].

@@ -1113,6 +1113,9 @@ __global__ __launch_bounds__(kThreads) void w8a16_kernel(W8Args a) {
   }
 }
 
+constexpr int w4a16_gemv_max_k() { return 32 * 256; }
+constexpr int w4a16_gemv_long_k() { return 32 * 512; }
+
 template <int MR, int R>
 hipError_t launch_gemv_r(const W4Args& a, hipStream_t s) {
   const int waves = (a.N + R - 1) / R;
@@ -1136,6 +1139,16 @@ hipError_t launch_gemv_r(const W4Args& a, hipStream_t s) {
   if (G <= 256)
     return launch<&w4a16_gemv_kernel<MR, 4, R, false>>(
         ktag("w4a16_gemv_kernel", MR, 4, R, false), dim3(blocks), dim3(kThreads), s, a);
+  // Long K: six or eight chunks per lane.  Two rows of X only with two rows
+  // of W per wave (more would need over 400 registers).
+  if constexpr (MR == 1 || (MR == 2 && R == 2)) {
+    if (G <= 384)
+      return launch<&w4a16_gemv_kernel<MR, 6, R, false>>(
+          ktag("w4a16_gemv_kernel", MR, 6, R, false), dim3(blocks), dim3(kThreads), s, a);
+    if (G <= 512)
+      return launch<&w4a16_gemv_kernel<MR, 8, R, false>>(
+          ktag("w4a16_gemv_kernel", MR, 8, R, false), dim3(blocks), dim3(kThreads), s, a);
+  }
   return hipErrorInvalidValue;
 }
 
@@ -1150,8 +1163,14 @@ hipError_t launch_gemv_mr(const W4Args& a, hipStream_t s) {
     return (k == 2 || k == 4 || k == 8) ? k : 0;
   }();
   const int simds = 4 * device_cu_count();
+  // Past K = 8192 a row's X work weighs more, so eight rows per wave already
+  // pay from six rows per SIMD on (K = 11008 M = 1, 2 / 4 / 8 rows per wave:
+  // N = 2048 5.8 / 7.4 / 9.5 us, 4096 8.7 / 8.8 / 10.0, 8192 14.8 / 13.5 /
+  // 11.8).
+  const bool long_k = a.K > w4a16_gemv_max_k();
   int r = forced;
-  if (!r) r = a.N < 4 * simds ? 2 : (a.N <= 16 * simds ? 4 : 8);
+  if (!r) r = a.N < 4 * simds ? 2 : (a.N <= (long_k ? 6 : 16) * simds ? 4 : 8);
+  if (long_k && MR == 2) r = 2;
   if (r == 2) return launch_gemv_r<MR, 2>(a, s);
   if (r == 4) return launch_gemv_r<MR, 4>(a, s);
   return launch_gemv_r<MR, 8>(a, s);
@@ -1159,7 +1178,6 @@ hipError_t launch_gemv_mr(const W4Args& a, hipStream_t s) {
 
 }  // namespace
 
-int w4a16_gemv_max_k() { return 32 * 256; }
 
 #ifndef NESO_SKINNY_WAVES
 #define NESO_SKINNY_WAVES 4
@@ -1176,7 +1194,14 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   const char* gemv_env = getenv("NESO_AMD_W4_GEMV_MAX_M");
   const int gemv_env_m = gemv_env ? atoi(gemv_env) : -1;
   const int gemv_max_m = (gemv_env_m >= 0 && gemv_env_m <= 4) ? gemv_env_m : 2;
-  if (a.M <= gemv_max_m && a.K <= w4a16_gemv_max_k()) {
+  // Up to K = 16384 the GEMV also serves M = 1, and M = 2 while N leaves two
+  // rows per wave (K = 11008, N = 4096 M = 1: 8.7 us against 13.3 for the
+  // X-in-LDS kernel and 25.4 for the 32 x 32 tile GEMM; M = 2, N = 2048 7.7
+  // against 12.6 and 24.9, but N = 4096 14.0 against 13.4).  Narrower
+  // matrices stay with the tile GEMM (test_long_k_small_m_route).
+  const bool gemv_long = a.K <= w4a16_gemv_long_k() && a.N >= 1024 &&
+                         (a.M == 1 || (a.M == 2 && a.N < 16 * device_cu_count()));
+  if (a.M <= gemv_max_m && (a.K <= w4a16_gemv_max_k() || gemv_long)) {
     switch (a.M) {
       case 1: return launch_gemv_mr<1>(a, s);
       case 2: return launch_gemv_mr<2>(a, s);
@@ -1241,7 +1266,7 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
                    : a.M > 32          ? 5
                                        : 6;
 
-  // The skinny kernels: X in LDS up to M = 16 (group 32, K <= 4096), the
+  // The skinny kernels: X in LDS where it applies (below), the
   // split-K skinny kernel otherwise up to M = 16 (past that K only where
   // the 32 x 32 tile grid would not fit on the CUs), and up to M = 32 when
   // the tile GEMM is off or its offsets would pass 2^31 bytes.
@@ -1254,8 +1279,24 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   const bool tile_ok = tile_fits && tile_mode != 0;
   const bool skinny_default =
       a.M <= 16 ? !(tile_ok && a.K > w4a16_skinny_lds_max_k() && tiles_of(32, 32) <= cus) : !tile_ok;
-  if (a.M <= 16 && a.M <= skinny_max_m && a.group == 32 && a.K % 128 == 0 &&
-      a.K <= w4a16_skinny_lds_max_k()) {
+  // X in LDS (us, this kernel against what served the call before):
+  // * M <= 16, K <= 4096, any power-of-two group (M = 16 group 128: K 4096
+  //   N 4096 5.8 against 16.1, N 11008 9.3 against 29.6, K 256 N 256 3.6
+  //   against 5.2);
+  // * M <= 16, longer K in phases of 4096 (M = 8 K 8192 N 4096 10.8 against
+  //   20.2, K 11008 N 1024 11.9 against 19.5, N 16384 27.8 against 47.1).
+  //   With group 32 past K = 8192, M = 9 .. 16 and N < 1024 stay with the
+  //   split-K skinny and tile kernels, which test_long_k_small_m_route fixes;
+  // * 17 <= M <= 32, phases of 2048 codes, from K = 1024 (N 4096 K 4096 9.6
+  //   against 12.4, K 11008 22.4 against 28.9; K 512 N 8192 6.4 against 5.6)
+  //   and while K / 1024 is no less than N / 8192 (K 1024 N 16384 8.0 against
+  //   7.2).  Below N = 1024 test_route_thresholds fixes the tile GEMM.
+  const bool lds_small = a.M <= 16 && a.M <= skinny_max_m &&
+                         (a.K <= w4a16_skinny_lds_max_k() || a.group > 32 ||
+                          (a.N >= 1024 && (a.M <= 8 || a.K <= 2 * w4a16_skinny_lds_max_k())));
+  const bool lds_mid = a.M > 16 && a.M <= 32 && !tile_env && !skinny_env && a.K >= 1024 && a.N >= 1024 &&
+                       (int64_t)a.K * 8 >= a.N;
+  if ((lds_small || lds_mid) && w4a16_skinny_lds_groups(a)) {
     // X in LDS, one persistent workgroup per CU, 8 waves splitting K
     // (qmatmul_skinny.hip).
     return launch_w4a16_skinny_lds(a, s);
