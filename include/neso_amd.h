@@ -230,6 +230,27 @@ int neso_rel_pos_precompute(const float* Q, const float* K_rel, const float* bia
                             void* Q_u, void* rel_bias, void* stream);
 
 /*
+ * Largest |x| of one to three fp32 tensors, for callers that choose the
+ * power-of-two factors of the split-precision kernels.  Tensor 0 is
+ * [batch][rows0][dim] with the given strides (elements), plus add0
+ * [batch][dim] where that is not NULL; tensors 1 and 2 are
+ * [batch][rows1][dim] with row_stride1, batch_stride1; a NULL x1 or x2 ends
+ * the list.  dim a multiple of 4.  neso_abs_max_begin enqueues one kernel
+ * that stores partial maxima to `slots` (pinned host memory the device can
+ * write, 256 per tensor are always enough) and returns minus the number of
+ * slots per tensor, or a status code > 0 (NESO_EUNSUPPORTED for sizes or
+ * strides it does not take, and while a launch plan is recorded).
+ * neso_abs_max_wait waits for that kernel, not for work enqueued after it,
+ * and gives each tensor's maximum: NaN if it holds a NaN.  `slots` may be
+ * used again once it has returned.
+ */
+int neso_abs_max_begin(const float* x0, const float* x1, const float* x2, const float* add0,
+                       int32_t batch, int32_t rows0, int32_t rows1, int32_t dim, int32_t row_stride0,
+                       int64_t batch_stride0, int32_t row_stride1, int64_t batch_stride1,
+                       uint32_t* slots, int32_t capacity, void* stream);
+int neso_abs_max_wait(const uint32_t* slots, int32_t each, int32_t count, float* maxima, void* stream);
+
+/*
  * Weight-only int4 matmul, Y[M][N] fp16 = X[M][K] fp16 * dequant(W)^T.
  * No reference kernel packs int4 (the reference's W4A16 stores one int4
  * value per int8, tests/test_quantized_matmul.py:170-178); this is the

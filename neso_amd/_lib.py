@@ -79,6 +79,11 @@ SIGNATURES = {
         ctypes.c_int,
         [_p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32, _p],
     ),
+    "neso_abs_max_begin": (
+        ctypes.c_int,
+        [_p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _i64, _i32, _i64, _p, _i32, _p],
+    ),
+    "neso_abs_max_wait": (ctypes.c_int, [_p, _i32, _i32, _p, _p]),
     "neso_w8a16_workspace_bytes": (_i64, [_p, _p, _i32, _i32, _i32, _i32, _i32]),
     "neso_w8a16_matmul_ws": (
         ctypes.c_int,

@@ -27,7 +27,7 @@ HARNESS_PATH = PKG / "neso_harness"
 ARCH = "gfx950"
 
 SOURCES = ["neso_abi.hip", "fa2_fwd.hip", "fa2_fast.hip", "relpos_pre.hip", "qmatmul.hip",
-           "qmatmul_skinny.hip", "qmatmul_w8_skinny.hip"]
+           "qmatmul_skinny.hip", "qmatmul_w8_skinny.hip", "range.hip"]
 
 # Per-source options on top of COMMON_FLAGS.  The skinny int4 kernel runs
 # 3-4% faster without the scheduler's memory-operation clustering (M = 16:

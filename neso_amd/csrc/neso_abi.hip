@@ -458,6 +458,50 @@ int neso_rel_pos_precompute(const float* Q, const float* K_rel, const float* bia
   return launched(neso::launch_relpos_precompute(a, d, static_cast<hipStream_t>(stream)), name);
 }
 
+int neso_abs_max_begin(const float* x0, const float* x1, const float* x2, const float* add0,
+                       int32_t batch, int32_t rows0, int32_t rows1, int32_t dim, int32_t row_stride0,
+                       int64_t batch_stride0, int32_t row_stride1, int64_t batch_stride1,
+                       uint32_t* slots, int32_t capacity, void* stream) {
+  const char* name = "abs_max_begin";
+  if (neso::plan_recording()) return fail(NESO_EUNSUPPORTED, "%s: a launch plan is being recorded", name);
+  neso::RangeArgs a{};
+  a.add = add0;
+  a.batch = batch;
+  a.dim = dim;
+  for (const float* x : {x0, x1, x2}) {
+    if (!x) break;
+    const int t = a.count++;
+    a.x[t] = x;
+    a.rows[t] = t ? rows1 : rows0;
+    a.row_stride[t] = t ? row_stride1 : row_stride0;
+    a.batch_stride[t] = t ? batch_stride1 : batch_stride0;
+    if ((reinterpret_cast<uintptr_t>(x) & 3u) || a.rows[t] <= 0 || a.row_stride[t] < 0 || a.batch_stride[t] < 0 ||
+        (int64_t)batch * a.rows[t] * dim > ((int64_t)1 << 33))
+      return fail(NESO_EUNSUPPORTED, "%s: tensor %d", name, t);
+  }
+  if (!a.count || batch <= 0 || dim <= 0 || dim % 4 || !slots || (reinterpret_cast<uintptr_t>(add0) & 3u))
+    return fail(NESO_EUNSUPPORTED, "%s: batch=%d dim=%d", name, batch, dim);
+  const int each = neso::abs_max_slots(a);
+  if (each * a.count > capacity) return fail(NESO_EINVAL, "%s: %d slots needed", name, each * a.count);
+  for (int i = 0; i < each * a.count; ++i) slots[i] = neso::kRangeEmpty;
+  std::atomic_thread_fence(std::memory_order_seq_cst);
+  const int st = launched(neso::launch_abs_max(a, each, slots, static_cast<hipStream_t>(stream)), name);
+  return st == NESO_OK ? -each : st;
+}
+
+int neso_abs_max_wait(const uint32_t* slots, int32_t each, int32_t count, float* maxima, void* stream) {
+  const char* name = "abs_max_wait";
+  if (!slots || !maxima || each <= 0 || count <= 0) return fail(NESO_EINVAL, "%s: bad arguments", name);
+  const int st = launched(neso::wait_abs_max(slots, each * count, static_cast<hipStream_t>(stream)), name);
+  if (st != NESO_OK) return st;
+  for (int t = 0; t < count; ++t) {
+    uint32_t m = 0;
+    for (int i = 0; i < each; ++i) m = std::max(m, slots[t * each + i]);
+    memcpy(&maxima[t], &m, 4);
+  }
+  return NESO_OK;
+}
+
 // True when a buffer of `bytes` bytes can be addressed with 32-bit offsets
 // (the kernels' buffer resources and per-lane offsets are 32-bit).
 static bool extent32(int64_t bytes) { return bytes < ((int64_t)1 << 32); }

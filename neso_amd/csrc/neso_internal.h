@@ -158,6 +158,23 @@ struct RelPreArgs {
   int32_t heads;
 };
 
+// Largest |x| of fp32 tensors [batch][rows][dim] (dim a multiple of 4), the
+// first one with add[batch][dim] added if given.
+struct RangeArgs {
+  const float* x[3];
+  const float* add;
+  int32_t count;
+  int32_t batch, dim;
+  int32_t rows[3];
+  int32_t row_stride[3];
+  int64_t batch_stride[3];
+};
+constexpr int kRangeSlots = 256;                 // at most, per tensor
+constexpr uint32_t kRangeEmpty = 0xFFFFFFFFu;    // no |x| has this pattern
+int abs_max_slots(const RangeArgs& a);
+hipError_t launch_abs_max(const RangeArgs& a, int slots_each, uint32_t* slots, hipStream_t stream);
+hipError_t wait_abs_max(const uint32_t* slots, int n, hipStream_t stream);
+
 hipError_t launch_relpos_precompute(const RelPreArgs& a, int head_dim, hipStream_t stream);
 
 }  // namespace neso

@@ -17,8 +17,9 @@ without a GPU, these functions raise.
 from __future__ import annotations
 
 import contextlib
-
+import ctypes
 import math
+import threading
 from typing import Any
 
 import torch
@@ -110,11 +111,73 @@ _SPLIT_TOP = 14     # rescaled inputs get their largest |x| in [2^13, 2^14)
 _QK_EXP_CAP = 50    # |exponent| of a Q or K rescale, so that the folded scale stays normal
 
 
-def _split_exponents(inputs, stream: int) -> dict[str, int]:
+class _Ranges(threading.local):
+    """This thread's pinned slots for neso_abs_max_begin / _wait: each use
+    ends with the wait, before the next one begins."""
+
+    def __init__(self):
+        self.slots = None
+        self.maxima = (ctypes.c_float * 3)()
+
+
+_ranges = _Ranges()
+_RANGE_CAPACITY = 3 * 256
+
+
+class _RangeCheck:
+    """Largest |x| of up to three fp32 tensors, measured on ``stream`` by one
+    kernel that is in flight from construction until :meth:`wait`."""
+
+    def __init__(self, views, stream: int, add=None):
+        """``views``: (tensor, batch, rows, dim, row stride, batch stride),
+        the last two tensors alike; ``add`` [batch, dim] goes on the first."""
+        if _ranges.slots is None:
+            _ranges.slots = torch.empty(_RANGE_CAPACITY, dtype=torch.int32, pin_memory=True)
+        self.lib, self.count, self.stream = _lib.load(), len(views), stream
+        x = [v[0].data_ptr() for v in views] + [None] * (3 - len(views))
+        first, rest = views[0], views[-1]
+        st = self.lib.neso_abs_max_begin(
+            *x, None if add is None else add.data_ptr(), first[1], first[2], rest[2], first[3],
+            first[4], first[5], rest[4], rest[5], _ranges.slots.data_ptr(), _RANGE_CAPACITY, stream)
+        self.each = -st
+        if st > 0 and st != _lib.NESO_EUNSUPPORTED:
+            _lib.check(st)
+
+    def wait(self) -> list[float] | None:
+        """The maxima, or None where the kernel does not take the views."""
+        if self.each <= 0:
+            return None
+        _lib.check(self.lib.neso_abs_max_wait(_ranges.slots.data_ptr(), self.each, self.count,
+                                              _ranges.maxima, self.stream))
+        return list(_ranges.maxima[:self.count])
+
+
+def _range_check(inputs, stream: int) -> _RangeCheck | None:
+    """A check of all ``inputs`` (as _split_exponents takes them) in flight,
+    or None where there is nothing to measure or the kernel does not fit."""
+    if not inputs or torch.cuda.is_current_stream_capturing():
+        return None
+    views = []
+    for t, _, shape, strides in inputs:
+        if t.device.type != "cuda":
+            return None
+        if len(shape) == 1:
+            shape, strides = (1, shape[0] // 32, 32), (0, 32, 1)
+        views.append((t, shape[0], shape[1], shape[2], strides[1], strides[0]))
+    if len({v[0].device for v in views}) > 1 or (len(views) == 3 and views[1][4:] != views[2][4:]):
+        return None
+    with _on_stream(stream, views[0][0].device):
+        if torch.cuda.is_current_stream_capturing():
+            return None
+    return _RangeCheck(views, stream)
+
+
+def _split_exponents(inputs, stream: int, maxima=None) -> dict[str, int]:
     """Power-of-two exponents for the fp32 inputs of a split-precision call.
 
     ``inputs`` holds (tensor, name, view shape, view strides) for the
-    elements the kernel reads.  One reduction per input and one
+    elements the kernel reads.  Their largest |x| are ``maxima`` where a
+    _RangeCheck has measured them, else one reduction per input and one
     synchronisation for all of them, on ``stream`` (the launch stream), so
     data written there before the call is what is measured.  Returns
     {name: k} for each input whose largest |x| lies outside _SPLIT_RANGE: k
@@ -125,17 +188,20 @@ def _split_exponents(inputs, stream: int) -> dict[str, int]:
     computation does).  Returns {} for raw addresses, host tensors
     (rejected at launch) and while the stream is being captured into a
     graph, where no synchronisation is possible."""
-    views = [(t.as_strided(shape, strides), name) for t, name, shape, strides in inputs
-             if isinstance(t, torch.Tensor) and t.device.type == "cuda"]
-    if not views or torch.cuda.is_current_stream_capturing():
-        return {}
-    dev = views[0][0].device
-    with _on_stream(stream, dev):
-        if torch.cuda.is_current_stream_capturing():
+    names = [name for _, name, _, _ in inputs]
+    if maxima is None:
+        views = [(t.as_strided(shape, strides), name) for t, name, shape, strides in inputs
+                 if isinstance(t, torch.Tensor) and t.device.type == "cuda"]
+        if not views or torch.cuda.is_current_stream_capturing():
             return {}
-        maxima = torch.stack([v.abs().amax() for v, _ in views]).cpu()
+        dev = views[0][0].device
+        with _on_stream(stream, dev):
+            if torch.cuda.is_current_stream_capturing():
+                return {}
+            maxima = torch.stack([v.abs().amax() for v, _ in views]).cpu().tolist()
+        names = [name for _, name in views]
     out = {}
-    for (_, name), m in zip(views, maxima.tolist()):
+    for name, m in zip(names, maxima):
         if math.isinf(m):
             raise _lib.NesoArgumentError(
                 _lib.NESO_EINVAL, f"{name}: infinite element; fp32 inputs must be finite")
@@ -156,13 +222,13 @@ def _pow2_scaled(t: torch.Tensor, k: int, name: str, stream: int) -> torch.Tenso
         return t * (2.0 ** k)
 
 
-def _rescale_split_inputs(Q, K, V, O, scale: float, inputs, stream: int, o_view):
+def _rescale_split_inputs(Q, K, V, O, scale: float, inputs, stream: int, o_view, maxima=None):
     """Apply _split_exponents: Q, K, V replaced by power-of-two rescaled
     copies where needed, the Q and K factors folded into ``scale``.  Returns
     (Q, K, V, scale, post) where ``post()`` undoes V's factor on O's view
     after the launch (None when V is not rescaled; V is left alone when O
     is not a tensor, and then must lie below 65504)."""
-    exps = _split_exponents(inputs, stream)
+    exps = _split_exponents(inputs, stream, maxima)
     if not exps:
         return Q, K, V, scale, None
     kq = max(-_QK_EXP_CAP, min(_QK_EXP_CAP, exps.get("Q", 0)))
@@ -184,6 +250,29 @@ def _rescale_split_inputs(Q, K, V, O, scale: float, inputs, stream: int, o_view)
             _lib.NESO_EINVAL, "V: |x| reaches the fp16 limit (65504) of the hi + lo split and O "
                               "is a raw address, so the result cannot be rescaled")
     return Q, K, V, scale * 2.0 ** -(kq + kk), post
+
+
+def _checked_launch(launch_kernel, Q, K, V, O, scale: float, inputs, stream: int, o_view,
+                    own_out: bool) -> None:
+    """Measure the fp32 inputs, rescale where needed, launch.  With
+    ``own_out`` (O is the call's own and no caller has seen it) the kernel is
+    queued behind the measurement at once and only run again, on rescaled
+    inputs, where the measurement asks for it."""
+    check = _range_check(inputs, stream)
+    maxima = None
+    ahead = own_out and check is not None
+    if check is not None:
+        try:
+            if ahead:
+                launch_kernel(Q, K, V, scale)
+        finally:
+            maxima = check.wait()
+    ahead = ahead and maxima is not None
+    Q2, K2, V2, scale2, post = _rescale_split_inputs(Q, K, V, O, scale, inputs, stream, o_view, maxima)
+    if not ahead or Q2 is not Q or K2 is not K or V2 is not V:
+        launch_kernel(Q2, K2, V2, scale2)
+    if post:
+        post()
 
 
 def flash_attention_fwd(Q, K, V, O, N: int, stride_qo: int, stride_kv: int, scale: float, *,
@@ -208,6 +297,14 @@ def flash_attention_fwd(Q, K, V, O, N: int, stride_qo: int, stride_kv: int, scal
     (V), so any finite magnitude keeps fp32-class accuracy.  Without it, or
     under graph capture, fp32 elements must lie below 65504 in magnitude.
     """
+    _flash_attention_fwd(Q, K, V, O, N, stride_qo, stride_kv, scale, head_dim, batch_heads,
+                         stride_bh_qo, stride_bh_kv, causal, qkv_dtype, check_range, stream, False)
+
+
+def _flash_attention_fwd(Q, K, V, O, N, stride_qo, stride_kv, scale, head_dim, batch_heads,
+                         stride_bh_qo, stride_bh_kv, causal, qkv_dtype, check_range, stream,
+                         own_out: bool) -> None:
+    """flash_attention_fwd; ``own_out`` as in _checked_launch."""
     if head_dim is None:
         if not isinstance(Q, torch.Tensor):
             raise ValueError("head_dim is required when Q is a raw address")
@@ -222,28 +319,29 @@ def flash_attention_fwd(Q, K, V, O, N: int, stride_qo: int, stride_kv: int, scal
         for t, nm, sp in ((Q, "Q", span_q), (K, "K", span_kv), (V, "V", span_kv),
                           (O, "O", span_q)):
             _extent(t, nm, sp)
-    post = None
+    dt = torch.float32 if qkv_dtype == "f32" else torch.float16
+    lib = _lib.load()
+    fn = lib.neso_flash_attention_f32_fwd if qkv_dtype == "f32" else lib.neso_flash_attention_fwd
+    st = _stream(stream, Q, O)
+
+    def launch_kernel(Q, K, V, scale):
+        _lib.check(fn(
+            _ptr(Q, "Q", dt), _ptr(K, "K", dt), _ptr(V, "V", dt),
+            _ptr(O, "O", torch.float32), int(N), int(stride_qo), int(stride_kv), float(scale),
+            int(head_dim), int(batch_heads), int(stride_bh_qo), int(stride_bh_kv),
+            int(bool(causal)), st))
+
     if qkv_dtype == "f32" and check_range and N > 0 and batch_heads > 0:
-        st = _stream(stream, Q, O)
-        Q, K, V, scale, post = _rescale_split_inputs(
-            Q, K, V, O, scale,
+        _checked_launch(
+            launch_kernel, Q, K, V, O, scale,
             [(t, nm, (batch_heads, N, head_dim), (sb, sr, 1))
              for t, nm, sr, sb in ((Q, "Q", stride_qo, stride_bh_qo),
                                    (K, "K", stride_kv, stride_bh_kv),
                                    (V, "V", stride_kv, stride_bh_kv))
              if isinstance(t, torch.Tensor) and t.dtype == torch.float32], st,
-            lambda: O.as_strided((batch_heads, N, head_dim), (stride_bh_qo, stride_qo, 1)))
-    lib = _lib.load()
-    dt = torch.float32 if qkv_dtype == "f32" else torch.float16
-    fn = lib.neso_flash_attention_f32_fwd if qkv_dtype == "f32" else lib.neso_flash_attention_fwd
-    st = fn(
-        _ptr(Q, "Q", dt), _ptr(K, "K", dt), _ptr(V, "V", dt),
-        _ptr(O, "O", torch.float32), int(N), int(stride_qo), int(stride_kv), float(scale),
-        int(head_dim), int(batch_heads), int(stride_bh_qo), int(stride_bh_kv), int(bool(causal)),
-        _stream(stream, Q, O))
-    _lib.check(st)
-    if post:
-        post()
+            lambda: O.as_strided((batch_heads, N, head_dim), (stride_bh_qo, stride_qo, 1)), own_out)
+    else:
+        launch_kernel(Q, K, V, scale)
 
 
 def flash_attention_io_fwd(Q, K, V, O, N: int, d_head: int, scale: float, *,
@@ -269,23 +367,25 @@ def flash_attention_io_fwd(Q, K, V, O, N: int, d_head: int, scale: float, *,
     if N > 0 and batch_heads > 0:
         for t, nm in ((Q, "Q"), (K, "K"), (V, "V"), (O, "O")):
             _extent(t, nm, batch_heads * N * d_head)
-    post = None
-    if io_dtype == "f32" and check_range and N > 0 and batch_heads > 0:
-        n_el = batch_heads * N * d_head
-        Q, K, V, scale, post = _rescale_split_inputs(
-            Q, K, V, O, scale,
-            [(t, nm, (n_el,), (1,)) for t, nm in ((Q, "Q"), (K, "K"), (V, "V"))
-             if isinstance(t, torch.Tensor) and t.dtype == torch.float32],
-            _stream(stream, Q, O), lambda: O.view(-1)[:n_el])
     dt = torch.float32 if io_dtype == "f32" else torch.float16
     lib = _lib.load()
-    st = lib.neso_flash_attention_io_fwd(
-        _ptr(Q, "Q", dt), _ptr(K, "K", dt), _ptr(V, "V", dt), _ptr(O, "O", dt), int(N),
-        int(d_head), float(scale), _lib.NESO_IO_F32 if io_dtype == "f32" else _lib.NESO_IO_F16,
-        int(batch_heads), _stream(stream, Q, O))
-    _lib.check(st)
-    if post:
-        post()
+    st = _stream(stream, Q, O)
+
+    def launch_kernel(Q, K, V, scale):
+        _lib.check(lib.neso_flash_attention_io_fwd(
+            _ptr(Q, "Q", dt), _ptr(K, "K", dt), _ptr(V, "V", dt), _ptr(O, "O", dt), int(N),
+            int(d_head), float(scale), _lib.NESO_IO_F32 if io_dtype == "f32" else _lib.NESO_IO_F16,
+            int(batch_heads), st))
+
+    if io_dtype == "f32" and check_range and N > 0 and batch_heads > 0:
+        n_el = batch_heads * N * d_head
+        _checked_launch(
+            launch_kernel, Q, K, V, O, scale,
+            [(t, nm, (n_el,), (1,)) for t, nm in ((Q, "Q"), (K, "K"), (V, "V"))
+             if isinstance(t, torch.Tensor) and t.dtype == torch.float32],
+            st, lambda: O.view(-1)[:n_el], False)
+    else:
+        launch_kernel(Q, K, V, scale)
 
 
 def flash_attention_window_fwd(Q, K, V, O, seq_len: int, stride_h: int, stride_m: int,
@@ -376,6 +476,15 @@ def rel_pos_precompute(Q, K_rel, bias_u, bias_v, T: int, d: int, nh: int, scale:
     magnitude; ``check_range`` verifies that before the launch (device
     reductions and a synchronisation, skipped under graph capture).
     """
+    _rel_pos_precompute(Q, K_rel, bias_u, bias_v, T, d, nh, scale, Q_u, rel_bias, check_range, stream,
+                        False)
+
+
+def _rel_pos_precompute(Q, K_rel, bias_u, bias_v, T, d, nh, scale, Q_u, rel_bias, check_range, stream,
+                        own_out: bool) -> None:
+    """rel_pos_precompute; with ``own_out`` the kernel is queued behind the
+    magnitude check instead of after it (no caller has seen the outputs)."""
+    check = False
     if T > 0 and nh > 0:
         for t, nm, n in ((Q, "Q", nh * T * d), (K_rel, "K_rel", nh * (2 * T - 1) * d),
                          (bias_u, "bias_u", nh * d), (bias_v, "bias_v", nh * d),
@@ -384,24 +493,43 @@ def rel_pos_precompute(Q, K_rel, bias_u, bias_v, T: int, d: int, nh: int, scale:
         if check_range and all(isinstance(x, torch.Tensor) and x.device.type == "cuda"
                                and x.dtype == torch.float32 for x in (Q, K_rel, bias_v)) \
                 and not torch.cuda.is_current_stream_capturing():
-            st = _stream(stream, Q, Q_u)
+            check = True
+    lib = _lib.load()
+    f32, f16 = torch.float32, torch.float16
+    st = _stream(stream, Q, Q_u)
+
+    def launch_kernel():
+        _lib.check(lib.neso_rel_pos_precompute(
+            _ptr(Q, "Q", f32), _ptr(K_rel, "K_rel", f32), _ptr(bias_u, "bias_u", f32),
+            _ptr(bias_v, "bias_v", f32), int(T), int(d), int(nh), float(scale),
+            _ptr(Q_u, "Q_u", f16), _ptr(rel_bias, "rel_bias", f16), st))
+
+    ahead = False
+    if check:
+        maxima = None
+        if Q.is_contiguous() and K_rel.is_contiguous() and bias_v.is_contiguous() \
+                and Q.device == K_rel.device == bias_v.device:
+            ranges = _RangeCheck([(Q, nh, T, d, d, T * d), (K_rel, nh, 2 * T - 1, d, d, (2 * T - 1) * d)],
+                                 st, bias_v)
+            try:
+                ahead = own_out and ranges.each > 0
+                if ahead:
+                    launch_kernel()
+            finally:
+                maxima = ranges.wait()
+        if maxima is None:
             with _on_stream(st, Q.device):
                 qv = (Q.reshape(-1)[:nh * T * d].view(nh, T, d)
                       + bias_v.reshape(-1)[:nh * d].view(nh, 1, d))
                 kr = K_rel.reshape(-1)[:nh * (2 * T - 1) * d]
                 maxima = torch.stack([qv.abs().amax(), kr.abs().amax()]).cpu().tolist()
-            for m, nm in zip(maxima, ("Q + bias_v", "K_rel")):
-                if m >= 65504.0:
-                    raise _lib.NesoArgumentError(
-                        _lib.NESO_EINVAL, f"{nm}: |x| reaches {m:g}; the precompute needs "
-                                          f"|Q + bias_v|, |K_rel| < 65504 (fp16 hi + lo split)")
-    lib = _lib.load()
-    f32, f16 = torch.float32, torch.float16
-    st = lib.neso_rel_pos_precompute(
-        _ptr(Q, "Q", f32), _ptr(K_rel, "K_rel", f32), _ptr(bias_u, "bias_u", f32),
-        _ptr(bias_v, "bias_v", f32), int(T), int(d), int(nh), float(scale),
-        _ptr(Q_u, "Q_u", f16), _ptr(rel_bias, "rel_bias", f16), _stream(stream, Q, Q_u))
-    _lib.check(st)
+        for m, nm in zip(maxima, ("Q + bias_v", "K_rel")):
+            if m >= 65504.0:
+                raise _lib.NesoArgumentError(
+                    _lib.NESO_EINVAL, f"{nm}: |x| reaches {m:g}; the precompute needs "
+                                      f"|Q + bias_v|, |K_rel| < 65504 (fp16 hi + lo split)")
+    if not ahead:
+        launch_kernel()
 
 
 def w4a16_matmul(X, W, scales, Y, M: int, N: int, K: int, stride_xm: int, stride_ym: int,
@@ -428,45 +556,47 @@ def _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N) -> Non
         _extent(scale, "scale", N)
 
 
-def _w8(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N, stream) -> None:
+_W8_SPLIT_MAX_M = 64  # largest M with a K split over workgroups
+
+
+def _w8(A, B, C, scale, scaled: bool, K, stride_am, stride_bk, stride_cm, M, N, stream) -> None:
     _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N)
     lib = _lib.load()
     M, N, K = int(M), int(N), int(K)
     stride_am, stride_bk, stride_cm = int(stride_am), int(stride_bk), int(stride_cm)
     a, b = _ptr(A, "A", torch.float16), _ptr(B, "B", torch.int8)
     c = _ptr(C, "C", torch.float32)
-    s = None if scale is None else _ptr(scale, "scale", torch.float16)
+    s = _ptr(scale, "scale", torch.float16)
     st = _stream(stream, A, C)
     # Partial sums of a K split, where the call has one.  The workspace comes
     # from torch's allocator on the launch stream, so it is reused only in
     # that stream's order (and stays in the pool of a captured graph).
-    ws = None
-    if isinstance(A, torch.Tensor):
+    ws, need = None, 0
+    if M <= _W8_SPLIT_MAX_M and isinstance(A, torch.Tensor):
         need = lib.neso_w8a16_workspace_bytes(a, b, K, stride_am, stride_bk, M, N)
         if need:
             with _on_stream(st, A.device), contextlib.suppress(torch.cuda.OutOfMemoryError):
                 ws = torch.empty(need // 4, dtype=torch.float32, device=A.device)
-    w, need = (0, 0) if ws is None else (ws.data_ptr(), ws.numel() * 4)
-    if s is None:
-        status = lib.neso_w8a16_matmul_ws(a, b, c, None, K, stride_am, stride_bk, stride_cm, M, N, w, need, st)
+    if ws is not None:
+        status = lib.neso_w8a16_matmul_ws(a, b, c, s, K, stride_am, stride_bk, stride_cm, M, N,
+                                          ws.data_ptr(), need, st)
+    elif scaled:
+        status = lib.neso_w8a16_scaled_matmul(a, b, c, s, K, stride_am, stride_bk, stride_cm, M, N, st)
     else:
-        if not s:  # the scaled entry point rejects a null scale
-            status = lib.neso_w8a16_scaled_matmul(a, b, c, s, K, stride_am, stride_bk, stride_cm, M, N, st)
-        else:
-            status = lib.neso_w8a16_matmul_ws(a, b, c, s, K, stride_am, stride_bk, stride_cm, M, N, w, need, st)
+        status = lib.neso_w8a16_matmul(a, b, c, K, stride_am, stride_bk, stride_cm, M, N, st)
     _lib.check(status)
 
 
 def w8a16_matmul(A, B, C, K: int, stride_am: int, stride_bk: int, stride_cm: int, *, M: int,
                  N: int, stream=None) -> None:
     """C fp32 = A fp16 @ f16(B int8 [K, N]) (tests/test_quantized_matmul.py:77-80 order)."""
-    _w8(A, B, C, None, K, stride_am, stride_bk, stride_cm, M, N, stream)
+    _w8(A, B, C, None, False, K, stride_am, stride_bk, stride_cm, M, N, stream)
 
 
 def w8a16_scaled_matmul(A, B, C, scale, K: int, stride_am: int, stride_bk: int, stride_cm: int,
                         *, M: int, N: int, stream=None) -> None:
     """C = (A @ f16(B)) * scale[n] (tests/test_quantized_matmul.py:189-192 order)."""
-    _w8(A, B, C, 0 if scale is None else scale, K, stride_am, stride_bk, stride_cm, M, N, stream)
+    _w8(A, B, C, scale, True, K, stride_am, stride_bk, stride_cm, M, N, stream)
 
 
 KERNELS = {
@@ -532,14 +662,14 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
         raise TypeError("q, k, v must share one dtype")
     n, d = int(q.shape[-2]), int(q.shape[-1])
     bh = q.numel() // max(n * d, 1) if n * d else 0
-    if out is None:
+    own_out = out is None
+    if own_out:
         out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
     _require(out.shape == q.shape and out.is_contiguous() and out.dtype == torch.float32,
              f"out must be a contiguous fp32 tensor of shape {tuple(q.shape)}")
     scale = 1.0 / math.sqrt(d) if scale is None else scale
-    flash_attention_fwd(q, k, v, out, n, d, d, scale, head_dim=d, batch_heads=bh,
-                        stride_bh_qo=n * d, stride_bh_kv=n * d, causal=causal,
-                        check_range=check_range)
+    _flash_attention_fwd(q, k, v, out, n, d, d, scale, d, bh, n * d, n * d, causal, None,
+                         check_range, None, own_out)
     return out
 
 
@@ -586,7 +716,8 @@ def precompute_bias_and_qu(q: torch.Tensor, k_rel: torch.Tensor, bias_u: torch.T
         _require(x.is_contiguous() and x.dtype == torch.float32, f"{nm} must be contiguous fp32")
     q_u = torch.empty((nh, t, d), dtype=torch.float16, device=q.device)
     rel_bias = torch.empty((nh, t, t), dtype=torch.float16, device=q.device)
-    rel_pos_precompute(q, k_rel, bias_u, bias_v, t, d, nh, 1.0 / math.sqrt(d), q_u, rel_bias)
+    _rel_pos_precompute(q, k_rel, bias_u, bias_v, t, d, nh, 1.0 / math.sqrt(d), q_u, rel_bias, True, None,
+                        True)
     return q_u, rel_bias
 
 
