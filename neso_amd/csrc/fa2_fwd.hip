@@ -255,22 +255,36 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void fa2_fwd_kernel(Fa2Args p) {
   const int krow = kRowPerm(ql);
   const half2v ones = {(half_t)1.f, (half_t)1.f};
 
-  // Dense f16 bias (the reference's rel-pos mode) with every row 16-byte
-  // aligned (kBiasDenseF16Row16: N, the head stride and the base multiples
-  // of 8 halves): lane (ql, g) needs B[q][kb0 + 32 t + 16 h + 8 g + 0..7]
-  // for tile t and half h of a block, eight consecutive halves, one 16-byte
-  // load.  They are issued one step ahead into a two-block register ring
-  // (block i in slot i % 2), so their latency (the bias is read once, from
-  // HBM) overlaps the previous block's work.  Block indices are clamped
-  // like the K/V loads, so every step issues the same loads.  Rows and keys
-  // past N read zeros or the next row's values; every such key is masked.
-  // Unaligned rows (kBiasDenseF16) are read element by element when the
-  // scores are formed.
-  constexpr bool kDense = BIAS == kBiasDenseF16Row16;
-  half8v bb[kDense ? 2 : 1][kDense ? 2 * NT : 1];
-  const rsrc_t rsB = make_rsrc(
-      kDense ? static_cast<const half_t*>(p.bias) + (int64_t)bh * p.bias_stride_h : nullptr,
-      kDense ? (uint32_t)((int64_t)N * N * 2) : 0u);
+  // Dense f16 bias (the reference's rel-pos mode): lane (ql, g) needs
+  // B[q][kb0 + 32 t + 16 h + 8 g + 0..7] for tile t and half h of a block,
+  // eight consecutive halves: one 16-byte load where rows start on 4-byte
+  // boundaries (kBiasDenseF16), else a fifth dword, the eight halves then
+  // shifted out of the five by this row's parity (kBiasDenseF16Odd).  The loads are
+  // issued one step ahead into a two-block register ring (block i in slot
+  // i % 2), so their latency (the bias is read once, from HBM) overlaps the
+  // previous block's work.  Block indices are clamped like the K/V loads, so
+  // every step issues the same loads.  Rows and keys past N read zeros or
+  // the next row's values; every such key is masked.  Raw buffer loads are
+  // range-checked dword by dword, so a load that straddles the end still
+  // returns its valid part.  H8 d64, before (one 2-byte load per element
+  // when the scores are formed, unless rows are 16-byte aligned) and now:
+  // T = 1504 18.8 / 18.9 us, 1500 53.9 / 19.3, 1499 63.2 / 23.4; d128
+  // T = 511 31.9 / 17.2, 1500 90.6 / 34.9.
+  constexpr bool kDense = BIAS == kBiasDenseF16 || BIAS == kBiasDenseF16Odd;
+  constexpr bool kOdd = BIAS == kBiasDenseF16Odd;
+  uint4v bb[kDense ? 2 : 1][kDense ? 2 * NT : 1];
+  uint32_t bx[kOdd ? 2 : 1][kOdd ? 2 * NT : 1];  // the fifth dwords
+  // Rows q0 .. of this head, from the 4-byte boundary at or below them; the
+  // elements before row q0 are bpar (0 or 1).  The extent is rounded up to
+  // whole dwords.
+  const half_t* bias0 = kDense ? static_cast<const half_t*>(p.bias) + (int64_t)bh * p.bias_stride_h +
+                                     (int64_t)q0 * N
+                               : nullptr;
+  const uint32_t bpar = kOdd ? (uint32_t)(reinterpret_cast<uintptr_t>(bias0) >> 1) & 1u : 0u;
+  const rsrc_t rsB = make_rsrc(kDense ? bias0 - bpar : nullptr,
+                               kDense ? (uint32_t)((((int64_t)(N - q0) * N + bpar) * 2 + 3) & ~(int64_t)3) : 0u);
+  const uint32_t brow = (uint32_t)(q - q0) * (uint32_t)N + bpar + 8u * g;
+  const uint32_t bshift = kOdd ? 16u * (brow & 1u) : 0u;  // blocks start at even keys
   auto bias_load = [&](int i, int slot) {
     if constexpr (kDense) {
       const int kb0 = (blk0 + max(0, min(kgu + KSPLIT * i, nblk - 1))) * kKB;
@@ -278,10 +292,29 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void fa2_fwd_kernel(Fa2Args p) {
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+          const uint32_t off = (brow + (uint32_t)(kb0 + 32 * t + 16 * h)) * 2u;
           bb[slot][2 * t + h] =
-              buf_load_half8(rsB, (uint32_t)(q * N + kb0 + 32 * t + 16 * h + 8 * g) * 2u);
+              __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rsB, off & ~3u, 0, 0));
+          if constexpr (kOdd)
+            bx[slot][2 * t + h] = __builtin_amdgcn_raw_buffer_load_b32(rsB, (off & ~3u) + 16u, 0, 0);
         }
     }
+  };
+  // Halves r & 7 of chunk r >> 3 of tile t of the block in ring slot `slot`.
+  auto bias_at = [&](int slot, int t) {
+    half8v b[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      uint4v w = bb[slot][2 * t + h];
+      if constexpr (kOdd) {
+        const uint32_t x = bx[slot][2 * t + h];
+        w = uint4v{__builtin_amdgcn_alignbit(w[1], w[0], bshift), __builtin_amdgcn_alignbit(w[2], w[1], bshift),
+                   __builtin_amdgcn_alignbit(w[3], w[2], bshift), __builtin_amdgcn_alignbit(x, w[3], bshift)};
+      }
+      b[h] = __builtin_bit_cast(half8v, w);
+    }
+    struct Pair { half8v b[2]; };
+    return Pair{{b[0], b[1]}};
   };
 
   auto compute = [&](int i, int buf) {
@@ -313,27 +346,26 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void fa2_fwd_kernel(Fa2Args p) {
     // window of some query of this wave.
     const bool masked =
         (kb0 + kKB > N) || (CAUSAL && (kb0 + kKB - 1 > qw0 + wr || kb0 < qw0 + 31 - wl));
-    if (BIAS != kBiasNone) {
+    if constexpr (kDense) {
+      // Reference semantics: (QK^T + B) * scale, B dense [T, T] f16 (keys past
+      // N are masked below).
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const auto bt = bias_at(buf, t);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float b = (float)bt.b[r >> 3][r & 7];
+          s[t][r] = (s[t][r] + (neg ? -b : b)) * c;
+        }
+      }
+    } else if constexpr (BIAS != kBiasNone) {
+      // BASELINE semantics: QK^T * scale + table[h][q - key + N - 1].
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int kr = 32 * t + 16 * (r >> 3) + 8 * g + (r & 7);  // key - kb0
-          if constexpr (kDense) {
-            // Reference semantics: (QK^T + B) * scale, B dense [T, T] f16
-            // (prefetched by bias_load; keys past N are masked below).
-            const float b = (float)(buf ? bb[1][2 * t + (r >> 3)][r & 7] : bb[0][2 * t + (r >> 3)][r & 7]);
-            s[t][r] = (s[t][r] + (neg ? -b : b)) * c;
-          } else if constexpr (BIAS == kBiasDenseF16) {
-            const int key = kb0 + kr;
-            const half_t* bp = static_cast<const half_t*>(p.bias) +
-                               (int64_t)bh * p.bias_stride_h;
-            const float b = (q < N && key < N) ? (float)bp[(int64_t)q * N + key] : 0.f;
-            s[t][r] = (s[t][r] + (neg ? -b : b)) * c;
-          } else {
-            // BASELINE semantics: QK^T * scale + table[h][q - key + N - 1].
-            s[t][r] = __builtin_fmaf(s[t][r], c, sBias[kg][buf][(q - q0) - kr + (kKB - 1)]);
-          }
+          s[t][r] = __builtin_fmaf(s[t][r], c, sBias[kg][buf][(q - q0) - kr + (kKB - 1)]);
         }
       }
     }
@@ -697,14 +729,13 @@ hipError_t launch_fa2(Fa2Args a, int head_dim, bool causal, int bias_kind, bool 
     return out_f16 ? launch_fa2_d<kBiasTableF32, true>(a, head_dim, causal, ksplit, stream)
                    : launch_fa2_d<kBiasTableF32, false>(a, head_dim, causal, ksplit, stream);
   }
-  // Dense bias rows that all start 16-byte aligned take 16-byte loads (the
-  // kernel forms 32-bit offsets into one head's N x N bias: N <= 32768).
-  if (a.N % 8 == 0 && a.N <= 32768 && a.bias_stride_h % 8 == 0 &&
-      (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0)
-    return out_f16 ? launch_fa2_d<kBiasDenseF16Row16, true>(a, head_dim, causal, ksplit, stream)
-                   : launch_fa2_d<kBiasDenseF16Row16, false>(a, head_dim, causal, ksplit, stream);
-  return out_f16 ? launch_fa2_d<kBiasDenseF16, true>(a, head_dim, causal, ksplit, stream)
-                 : launch_fa2_d<kBiasDenseF16, false>(a, head_dim, causal, ksplit, stream);
+  // Dense bias rows that all start on 4-byte boundaries take plain 16-byte
+  // loads.
+  if (a.N % 2 == 0 && a.bias_stride_h % 2 == 0 && (reinterpret_cast<uintptr_t>(a.bias) & 3) == 0)
+    return out_f16 ? launch_fa2_d<kBiasDenseF16, true>(a, head_dim, causal, ksplit, stream)
+                   : launch_fa2_d<kBiasDenseF16, false>(a, head_dim, causal, ksplit, stream);
+  return out_f16 ? launch_fa2_d<kBiasDenseF16Odd, true>(a, head_dim, causal, ksplit, stream)
+                 : launch_fa2_d<kBiasDenseF16Odd, false>(a, head_dim, causal, ksplit, stream);
 }
 
 }  // namespace neso

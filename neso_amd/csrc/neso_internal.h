@@ -10,9 +10,9 @@
 
 namespace neso {
 
-// kBiasDenseF16Row16 is internal to the generic FA2 kernel: the dense f16
-// bias with every row 16-byte aligned (16-byte bias loads).
-enum BiasKind { kBiasNone = 0, kBiasTableF32 = 1, kBiasDenseF16 = 2, kBiasDenseF16Row16 = 3 };
+// kBiasDenseF16Odd is internal to the generic FA2 kernel: the dense f16 bias
+// with rows that do not all start on 4-byte boundaries.
+enum BiasKind { kBiasNone = 0, kBiasTableF32 = 1, kBiasDenseF16 = 2, kBiasDenseF16Odd = 3 };
 
 struct Fa2Args {
   const void* Q;        // f16, or f32 for the f32-input kernels
