@@ -1237,7 +1237,7 @@ constexpr char kManifest[] = R"JSON({
      "template_params": [
       "T"
      ],
-     "when": "M > 64, K, N, lda, ldb multiples of 8 and A 16-byte / B 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64)",
+     "when": "M > 64, or K, N, lda, ldb not multiples of 8 or A not 16-byte / B not 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when aligned and cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64); with a workspace (neso_w8a16_matmul_ws) grid z splits K and w8a16_reduce_kernel follows",
      "threadgroup_size": "2 * T",
      "num_warps": "T // 32",
      "grid": [
@@ -1255,7 +1255,7 @@ constexpr char kManifest[] = R"JSON({
      "device_kernel": "w8a16_kernel",
      "source": "neso_amd/csrc/qmatmul.hip",
      "template_params": [],
-     "when": "any other shape or alignment",
+     "when": "256 rows of A or B of 2^31 bytes and more",
      "threadgroup_size": "256",
      "num_warps": "4",
      "grid": [
@@ -1382,7 +1382,7 @@ constexpr char kManifest[] = R"JSON({
      "template_params": [
       "T"
      ],
-     "when": "M > 64, K, N, lda, ldb multiples of 8 and A 16-byte / B 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64)",
+     "when": "M > 64, or K, N, lda, ldb not multiples of 8 or A not 16-byte / B not 8-byte aligned: T x T MFMA tiles, B dequantised into LDS as [k][n] f16 and read transposed; T = 256 (eight waves of 64 x 128) when aligned and cdiv(M, 256) * cdiv(N, 256) >= cus, else T = 128 (four waves of 64 x 64); with a workspace (neso_w8a16_matmul_ws) grid z splits K and w8a16_reduce_kernel follows",
      "threadgroup_size": "2 * T",
      "num_warps": "T // 32",
      "grid": [
@@ -1400,7 +1400,7 @@ constexpr char kManifest[] = R"JSON({
      "device_kernel": "w8a16_kernel",
      "source": "neso_amd/csrc/qmatmul.hip",
      "template_params": [],
-     "when": "any other shape or alignment",
+     "when": "256 rows of A or B of 2^31 bytes and more",
      "threadgroup_size": "256",
      "num_warps": "4",
      "grid": [

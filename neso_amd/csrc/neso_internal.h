@@ -131,13 +131,15 @@ struct W8Args {
   int32_t lda, ldb, ldc;
 };
 
-// Few rows of A (qmatmul_w8_skinny.hip), under w8a16_tiled's conditions:
-// M <= w8a16_skinny_max_m().  `splits` > 1 (at most w8a16_skinny_splits())
-// splits K over workgroups and needs a workspace of splits * M * N floats,
-// 16-byte aligned.
+// Few rows of A (qmatmul_w8_skinny.hip), with aligned operands: M <=
+// w8a16_skinny_max_m().  `splits` > 1 splits K over workgroups and needs a
+// workspace of splits * M * w8a16_part_stride(N) floats, 16-byte aligned.
 int w8a16_skinny_max_m();
 int w8a16_skinny_splits(const W8Args& a);
 hipError_t launch_w8a16_skinny(const W8Args& a, int splits, float* workspace, hipStream_t stream);
+// Row stride of partial sums, and their reduction into C.
+constexpr int w8a16_part_stride(int n) { return (n + 3) & ~3; }
+hipError_t launch_w8a16_reduce(const W8Args& a, int splits, const float* part, hipStream_t stream);
 
 // The workspace launch_w8a16 can use for this call, in bytes (0: none).
 int64_t w8a16_workspace_bytes(const W8Args& a);

@@ -926,10 +926,35 @@ __device__ __forceinline__ int w8_b_tr_offset(int lane, int hb, int u) {
   return w8_b_at(hb, row, cu >> 3) + (cu & 7);
 }
 
+// 16 bytes per lane at byte offset off of a buffer whose base is 4-byte
+// aligned, off on any boundary (UA) or on a 16-byte one: five dwords from
+// the boundary below, shifted when they are used.
+template <bool UA>
+struct Bytes16 {
+  uint4v d;
+  uint32_t e, shift;
+  __device__ __forceinline__ void load(rsrc_t r, uint32_t off, uint32_t oob) {
+    d = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(r, (UA ? off & ~3u : off) | oob, 0, 0));
+    if constexpr (UA) {
+      e = __builtin_amdgcn_raw_buffer_load_b32(r, ((off & ~3u) + 16u) | oob, 0, 0);
+      shift = 8u * (off & 3u);
+    }
+  }
+  __device__ __forceinline__ uint4v get() const {
+    if constexpr (!UA) return d;
+    return uint4v{__builtin_amdgcn_alignbit(d[1], d[0], shift), __builtin_amdgcn_alignbit(d[2], d[1], shift),
+                  __builtin_amdgcn_alignbit(d[3], d[2], shift), __builtin_amdgcn_alignbit(e, d[3], shift)};
+  }
+};
+
 // Workgroup tile T x T (T = 128: four waves of 64 x 64; T = 256: eight
 // waves of 64 x 128, a third fewer LDS bytes per MFMA), K-steps of kW8BK.
-template <int T>
-__global__ __launch_bounds__(2 * T) void w8a16_gemm_kernel(W8Args a) {
+// UA: any K, N, strides and alignment (M387 N978 K1623: 268 us with the
+// per-element kernel, 34 here, 20 with K split; M1000 K999 N1001 169 / 24).  part != nullptr: grid z splits the
+// K-steps into gridDim.z ranges, each workgroup storing its partial sums to
+// part[z][m][n] (rows of np floats) for w8a16_reduce_kernel.
+template <int T, bool UA>
+__global__ __launch_bounds__(2 * T) void w8a16_gemm_kernel(W8Args a, float* part, int32_t np) {
   constexpr int NT = 2 * T;          // threads
   constexpr int NI = T / 64;         // 32-column MFMA tiles per wave
   constexpr int NH = T / 128;        // 128-column B halves
@@ -950,12 +975,28 @@ __global__ __launch_bounds__(2 * T) void w8a16_gemm_kernel(W8Args a) {
   const int gm = min(mt - first, kGroupM), in = lid % (kGroupM * nt);
   const int m0 = (first + in % gm) * T, n0 = (in / gm) * T;
   const int mrows = min(T, a.M - m0);
+  // K range of this workgroup (T = 256 fills the chip and is never split).
+  constexpr bool kSplit = T == 128;
+  const int allsteps = (a.K + kW8BK - 1) / kW8BK;
+  const int per = kSplit ? (allsteps + (int)gridDim.z - 1) / (int)gridDim.z : allsteps;
+  const int kbeg = kSplit ? (int)blockIdx.z * per * kW8BK : 0;
+  const int kend = kSplit ? min(a.K, kbeg + per * kW8BK) : a.K;
+  const int nsteps = kSplit ? max(0, (kend - kbeg + kW8BK - 1) / kW8BK) : allsteps;
   constexpr uint32_t kOut = 0x80000000u;
-  const rsrc_t ra = make_rsrc(a.A + (int64_t)m0 * a.lda, (uint32_t)(((int64_t)(mrows - 1) * a.lda + a.K) * 2));
+  // Unaligned operands: the buffers start at the 4-byte boundary below, and
+  // their extents are rounded up to whole dwords (range checks are per
+  // dword).
+  const half_t* a0 = a.A + (int64_t)m0 * a.lda;
+  const int8_t* b0 = a.B + n0;
+  const uint32_t apar = UA ? (uint32_t)(reinterpret_cast<uintptr_t>(a0) & 3u) : 0u;
+  const uint32_t bpar = UA ? (uint32_t)(reinterpret_cast<uintptr_t>(b0) & 3u) : 0u;
+  auto whole = [](int64_t bytes) { return (uint32_t)(UA ? (bytes + 3) & ~(int64_t)3 : bytes); };
+  const rsrc_t ra = make_rsrc(reinterpret_cast<const char*>(a0) - apar,
+                              whole(((int64_t)(mrows - 1) * a.lda + a.K) * 2 + apar));
   // K >= 1 (the ABI rejects K = 0 with a non-empty output); the extent is
   // clamped at 0 anyway so a bad call cannot wrap it to ~4 GiB.
   const rsrc_t rb = make_rsrc(
-      a.B + n0, (uint32_t)max((int64_t)0, (a.K - 1) * (int64_t)a.ldb + min(T, a.N - n0)));
+      b0 - bpar, whole(max((int64_t)0, (a.K - 1) * (int64_t)a.ldb + min(T, a.N - n0) + bpar)));
   // A: rows ar + (T/2) j, 16-byte pieces ap + 4p of the step.
   const int ar = tid >> 2, ap = tid & 3;
   // B: k-row br of the step, columns 32 bc .. 32 bc + 31 (two 16-byte
@@ -965,29 +1006,39 @@ __global__ __launch_bounds__(2 * T) void w8a16_gemm_kernel(W8Args a) {
   const int br = tid / BG, bc = tid % BG;
   const uint32_t nlim = (uint32_t)min(T, a.N - n0);
   struct Stage {
-    half8v av[2][kW8AP];
-    uint4v b[2];  // 16 int8 of row br, columns 32 bc + 16 h ..
+    Bytes16<UA> av[2][kW8AP];
+    Bytes16<UA> b[2];  // 16 int8 of row br, columns 32 bc + 16 h ..
+    int left[UA ? kW8AP : 1];  // elements of the A piece before kend
   };
   auto load = [&](Stage& g, int k0) {
 #pragma unroll
     for (int p = 0; p < kW8AP; ++p) {
       const int kc = k0 + 8 * (ap + 4 * p);
-      const uint32_t aoob = kc < a.K ? 0u : kOut;
+      const uint32_t aoob = kc < kend ? 0u : kOut;
+      if constexpr (UA) g.left[p] = kend - kc;
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        g.av[j][p] = buf_load_half8(ra, (((uint32_t)(ar + (T / 2) * j) * a.lda + kc) * 2u) | aoob);
+        g.av[j][p].load(ra, ((uint32_t)(ar + (T / 2) * j) * a.lda + kc) * 2u + apar, aoob);
     }
-    // Pieces wholly past N are masked; a piece that straddles N (N % 16 =
-    // 8) reads bytes of columns >= N, whose products only reach columns of
-    // C that are never stored.  Rows past K fall outside the buffer.
+    // Pieces wholly past N are masked; a piece that straddles N reads bytes
+    // of columns >= N, whose products only reach columns of C that are never
+    // stored.  Rows past K fall outside the buffer.
     const int k = k0 + br;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const uint32_t col = 32u * bc + 16u * h;
-      g.b[h] = __builtin_bit_cast(
-          uint4v, __builtin_amdgcn_raw_buffer_load_b128(
-                      rb, ((uint32_t)k * a.ldb + col) | (k < a.K && col < nlim ? 0u : kOut), 0, 0));
+      g.b[h].load(rb, (uint32_t)k * a.ldb + col + bpar, k < kend && col < nlim ? 0u : kOut);
     }
+  };
+  // An A piece; past the end of the row it must hold zeros (the next row's
+  // elements, maybe not finite, would meet zero rows of B there).
+  auto apiece = [&](const Stage& g, int j, int p) {
+    uint4v w = g.av[j][p].get();
+    if constexpr (UA) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] &= g.left[p] > 2 * i + 1 ? ~0u : g.left[p] == 2 * i + 1 ? 0xFFFFu : 0u;
+    }
+    return __builtin_bit_cast(half8v, w);
   };
   const uint32_t magic = vgpr_const(0x64006400u);
   const half2v bias = {(half_t)1152, (half_t)1152};
@@ -996,15 +1047,16 @@ __global__ __launch_bounds__(2 * T) void w8a16_gemm_kernel(W8Args a) {
     for (int p = 0; p < kW8AP; ++p)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        as[buf][w8_a_at(ar + (T / 2) * j, ap + 4 * p) / 8] = g.av[j][p];
+        as[buf][w8_a_at(ar + (T / 2) * j, ap + 4 * p) / 8] = apiece(g, j, p);
     // Row br as f16 in [k][n] order: bytes (n, n+1) of a word -> one f16
     // pair; chunk c of the row at w8_b_at.
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       uint32_t pr[8];
+      const uint4v bw = g.b[h].get();
 #pragma unroll
       for (int wd = 0; wd < 4; ++wd) {
-        const uint32_t x = g.b[h][wd] ^ 0x80808080u;
+        const uint32_t x = bw[wd] ^ 0x80808080u;
         pr[2 * wd] = __builtin_amdgcn_perm(0u, x, 0x0c010c00u) | magic;
         pr[2 * wd + 1] = __builtin_amdgcn_perm(0u, x, 0x0c030c02u) | magic;
       }
@@ -1047,36 +1099,43 @@ __global__ __launch_bounds__(2 * T) void w8a16_gemm_kernel(W8Args a) {
     }
   };
 
-  const int nsteps = (a.K + kW8BK - 1) / kW8BK;
   Stage sA, sB;
-  load(sA, 0);
+  load(sA, kbeg);
   store(sA, 0);
-  load(sB, kW8BK);
+  load(sB, kbeg + kW8BK);
   lds_barrier();
   for (int st = 0; st < nsteps; st += 2) {
-    load(sA, (st + 2) * kW8BK);  // past K: zeros
+    load(sA, kbeg + (st + 2) * kW8BK);  // past kend: zeros
     compute(0);
     store(sB, 1);
     lds_barrier();
-    load(sB, (st + 3) * kW8BK);
+    load(sB, kbeg + (st + 3) * kW8BK);
     compute(1);
     store(sA, 0);
     lds_barrier();
   }
 
   // acc[mi][ni] register r: row 64wm + 32mi + 8(r/4) + 4(lane/32) + r%4,
-  // column (T/2) wn + 32ni + lane%32.
+  // column (T/2) wn + 32ni + lane%32.  Buffer stores: rows past M fall
+  // outside the buffer and columns past N get an offset outside it, so no
+  // element needs a branch or 64-bit address arithmetic (4096^3: 0.3% of
+  // 130 us).
+  const bool partial = kSplit && part;
+  float* c = partial ? part + (int64_t)blockIdx.z * a.M * np : a.C;
+  const uint32_t ldc = partial ? np : a.ldc;
+  const rsrc_t rc = make_rsrc(c + (int64_t)m0 * ldc + n0, ((uint32_t)(mrows - 1) * ldc + nlim) * 4u);
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni) {
-    const int n = n0 + (T / 2) * wn + 32 * ni + li;
-    if (n >= a.N) continue;
-    const float s = a.scale ? (float)a.scale[n] : 1.f;
+    const uint32_t col = (T / 2) * wn + 32 * ni + li;
+    const bool in_n = col < nlim;
+    const float s = a.scale && !partial && in_n ? (float)a.scale[n0 + col] : 1.f;
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = m0 + 64 * wm + 32 * mi + 8 * (r >> 2) + 4 * lh + (r & 3);
-        if (m < a.M) a.C[(int64_t)m * a.ldc + n] = acc[mi][ni][r] * s;
+        const uint32_t row = 64 * wm + 32 * mi + 8 * (r >> 2) + 4 * lh + (r & 3);
+        const uint32_t off = (row * ldc + col) * 4u | (in_n ? 0u : kOut);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[mi][ni][r] * s), rc, off, 0, 0);
       }
   }
 }
@@ -1369,42 +1428,78 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   return launch<&w4a16_mfma_kernel<TN>>(ktag("w4a16_mfma_kernel", TN), grid, dim3(kThreads), s, a);
 }
 
-// The tiled and skinny kernels read A and B in 16- and 8-byte pieces: A's
-// must be 16-byte aligned and never straddle the end of a row; B's need
-// 8-byte alignment (a 16-byte piece that straddles N reads columns that are
-// never stored).  Buffer offsets stay below 2^31 bytes.
-static bool w8a16_tiled(const W8Args& a) {
+// The skinny and the aligned tiled kernels read A and B in 16- and 8-byte
+// pieces: A's must be 16-byte aligned and never straddle the end of a row;
+// B's need 8-byte alignment (a 16-byte piece that straddles N reads columns
+// that are never stored).  All tiled kernels need buffer offsets below 2^31
+// bytes.
+static bool w8a16_aligned(const W8Args& a) {
   return a.K % 8 == 0 && a.lda % 8 == 0 && a.N % 8 == 0 && a.ldb % 8 == 0 &&
          (reinterpret_cast<uintptr_t>(a.A) & 15u) == 0 &&
-         (reinterpret_cast<uintptr_t>(a.B) & 7u) == 0 &&
-         (int64_t)256 * a.lda * 2 < ((int64_t)1 << 31) &&
-         (int64_t)a.K * a.ldb < ((int64_t)1 << 31);
+         (reinterpret_cast<uintptr_t>(a.B) & 7u) == 0;
+}
+static bool w8a16_offsets_fit(const W8Args& a) {
+  return (int64_t)256 * a.lda * 2 < ((int64_t)1 << 31) && (int64_t)(a.K + 256) * a.ldb < ((int64_t)1 << 31) &&
+         (int64_t)256 * a.ldc * 4 < ((int64_t)1 << 31);
+}
+static bool w8a16_skinny(const W8Args& a) { return a.M <= w8a16_skinny_max_m() && w8a16_aligned(a); }
+
+// K ranges of the 128 x 128-tile kernel, at most 16 and one workgroup per
+// CU: the count that saves most.  A K-step costs about 0.7 us whatever the
+// grid; the partial sums are written and read back (2e-6 us per element) and
+// the reduction is a launch of about 2.5 us.  us without and with the count
+// this gives: M128 K4096 N4096 46.0 / 21.1, M256 K4096 N4096 46.6 / 24.9,
+// M100 K4000 N304 44.6 / 12.1, M128 K1024 N1024 15.1 / 11.0; M1024 K1024
+// N1024 (15.8 against 17.2 with four) and M512 K512 N512 (10.0 against 11.1
+// with two) are not split.
+static int w8a16_tile_splits(const W8Args& a) {
+  const int64_t tiles = (int64_t)((a.N + 127) / 128) * ((a.M + 127) / 128);
+  const int steps = (a.K + kW8BK - 1) / kW8BK;
+  const int most = (int)min(min((int64_t)device_cu_count() / tiles, (int64_t)steps), (int64_t)16);
+  int best = 1;
+  double saved = 0.5;  // less is within the noise
+  for (int s = 2; s <= most; ++s) {
+    const double gain = 0.7 * (steps - (steps + s - 1) / s) - 2.5 - 2e-6 * s * a.M * a.N;
+    if (gain > saved) {
+      saved = gain;
+      best = s;
+    }
+  }
+  return best;
+}
+
+static int w8a16_splits(const W8Args& a) {
+  if (!w8a16_offsets_fit(a)) return 1;
+  return w8a16_skinny(a) ? w8a16_skinny_splits(a) : w8a16_tile_splits(a);
 }
 
 int64_t w8a16_workspace_bytes(const W8Args& a) {
-  if (a.M > w8a16_skinny_max_m() || !w8a16_tiled(a)) return 0;
-  const int splits = w8a16_skinny_splits(a);
-  return splits > 1 ? (int64_t)splits * a.M * a.N * 4 : 0;
+  const int splits = w8a16_splits(a);
+  return splits > 1 ? (int64_t)splits * a.M * w8a16_part_stride(a.N) * 4 : 0;
 }
 
 hipError_t launch_w8a16(const W8Args& a, void* workspace, int64_t workspace_bytes, hipStream_t s) {
-  const bool tiled = w8a16_tiled(a);
-  if (tiled && a.M <= w8a16_skinny_max_m()) {
+  if (w8a16_offsets_fit(a)) {
     const int64_t need = w8a16_workspace_bytes(a);
     const bool split = need && workspace && workspace_bytes >= need &&
                        (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
-    return launch_w8a16_skinny(a, split ? w8a16_skinny_splits(a) : 1, static_cast<float*>(workspace), s);
-  }
-  if (tiled) {
+    const int splits = split ? w8a16_splits(a) : 1;
+    float* part = splits > 1 ? static_cast<float*>(workspace) : nullptr;
+    const int np = w8a16_part_stride(a.N);
+    if (w8a16_skinny(a)) return launch_w8a16_skinny(a, splits, part, s);
     // 256 x 256 tiles (a third fewer LDS bytes per MFMA) when they still
     // give every CU a workgroup; 128 x 128 otherwise.
+    const bool aligned = w8a16_aligned(a);
     const int64_t big = (int64_t)((a.N + 255) / 256) * ((a.M + 255) / 256);
-    if (big >= device_cu_count()) {
+    if (aligned && big >= device_cu_count()) {
       const dim3 grid((a.N + 255) / 256, (a.M + 255) / 256);
-      return launch<&w8a16_gemm_kernel<256>>(ktag("w8a16_gemm_kernel", 256), grid, dim3(512), s, a);
+      return launch<&w8a16_gemm_kernel<256, false>>(ktag("w8a16_gemm_kernel", 256), grid, dim3(512), s, a, part, np);
     }
-    const dim3 grid((a.N + 127) / 128, (a.M + 127) / 128);
-    return launch<&w8a16_gemm_kernel<128>>(ktag("w8a16_gemm_kernel", 128), grid, dim3(256), s, a);
+    const dim3 grid((a.N + 127) / 128, (a.M + 127) / 128, splits);
+    const hipError_t e =
+        aligned ? launch<&w8a16_gemm_kernel<128, false>>(ktag("w8a16_gemm_kernel", 128), grid, dim3(256), s, a, part, np)
+                : launch<&w8a16_gemm_kernel<128, true>>(ktag("w8a16_gemm_kernel", 128), grid, dim3(256), s, a, part, np);
+    return e != hipSuccess || splits == 1 ? e : launch_w8a16_reduce(a, splits, part, s);
   }
   const dim3 grid((a.N + 127) / 128, (a.M + 31) / 32);
   return launch<&w8a16_kernel>(ktag("w8a16_kernel"), grid, dim3(kThreads), s, a);

@@ -157,13 +157,15 @@ __global__ __launch_bounds__(kWaves * kWave) void w8a16_skinny_kernel(W8Args a, 
 }
 
 // C[m][n] = scale[n] * sum over splits of part[s][m][n], in split order.
-__global__ __launch_bounds__(kWave) void w8a16_reduce_kernel(W8Args a, const float* part, int32_t splits) {
-  const int quads = a.N / 4;
+// Rows of part are w8a16_part_stride(N) floats.
+__global__ __launch_bounds__(kWave) void w8a16_reduce_kernel(W8Args a, const float* part, int32_t splits,
+                                                             int32_t np) {
+  const int quads = np / 4;
   const int64_t e = (int64_t)blockIdx.x * kWave + threadIdx.x;
   const int m = (int)(e / quads), n = 4 * (int)(e % quads);
   if (m >= a.M) return;
-  const int64_t mn = (int64_t)a.M * a.N;
-  const float* p = part + (int64_t)m * a.N + n;
+  const int64_t mn = (int64_t)a.M * np;
+  const float* p = part + (int64_t)m * np + n;
   // Eight loads at a time, the last batch clamped to the last partial.
   float4v v = float4v{};
   for (int s0 = 0; s0 < splits; s0 += 8) {
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(kWave) void w8a16_reduce_kernel(W8Args a, const flo
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    a.C[(int64_t)m * a.ldc + n + i] = v[i] * (a.scale ? (float)a.scale[n + i] : 1.f);
+    if (n + i < a.N) a.C[(int64_t)m * a.ldc + n + i] = v[i] * (a.scale ? (float)a.scale[n + i] : 1.f);
 }
 
 int mtiles(int m) { return m <= 16 ? 1 : m <= 32 ? 2 : 4; }
@@ -210,10 +212,14 @@ hipError_t launch_w8a16_skinny(const W8Args& a, int splits, float* workspace, hi
   hipError_t e = mt == 1   ? launch<&w8a16_skinny_kernel<1>>(tag, grid, block, s, a, part, splits)
                  : mt == 2 ? launch<&w8a16_skinny_kernel<2>>(tag, grid, block, s, a, part, splits)
                            : launch<&w8a16_skinny_kernel<4>>(tag, grid, block, s, a, part, splits);
-  if (e != hipSuccess || splits == 1) return e;
-  const int64_t quads = (int64_t)a.M * (a.N / 4);
-  return launch<&w8a16_reduce_kernel>(ktag("w8a16_reduce_kernel"), dim3((quads + kWave - 1) / kWave), dim3(kWave), s, a,
-                                      (const float*)workspace, splits);
+  return e != hipSuccess || splits == 1 ? e : launch_w8a16_reduce(a, splits, workspace, s);
+}
+
+hipError_t launch_w8a16_reduce(const W8Args& a, int splits, const float* part, hipStream_t s) {
+  const int np = w8a16_part_stride(a.N);
+  const int64_t quads = (int64_t)a.M * (np / 4);
+  return launch<&w8a16_reduce_kernel>(ktag("w8a16_reduce_kernel"), dim3((quads + kWave - 1) / kWave), dim3(kWave), s,
+                                      a, part, splits, np);
 }
 
 }  // namespace neso

@@ -556,7 +556,9 @@ def _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N) -> Non
         _extent(scale, "scale", N)
 
 
-_W8_SPLIT_MAX_M = 64  # largest M with a K split over workgroups
+# No call with a shorter K or more results splits K over workgroups (the
+# library decides for the others).
+_W8_SPLIT_MIN_K, _W8_SPLIT_MAX_MN = 512, 1 << 22
 
 
 def _w8(A, B, C, scale, scaled: bool, K, stride_am, stride_bk, stride_cm, M, N, stream) -> None:
@@ -572,7 +574,7 @@ def _w8(A, B, C, scale, scaled: bool, K, stride_am, stride_bk, stride_cm, M, N, 
     # from torch's allocator on the launch stream, so it is reused only in
     # that stream's order (and stays in the pool of a captured graph).
     ws, need = None, 0
-    if M <= _W8_SPLIT_MAX_M and isinstance(A, torch.Tensor):
+    if K >= _W8_SPLIT_MIN_K and M * N <= _W8_SPLIT_MAX_MN and isinstance(A, torch.Tensor):
         need = lib.neso_w8a16_workspace_bytes(a, b, K, stride_am, stride_bk, M, N)
         if need:
             with _on_stream(st, A.device), contextlib.suppress(torch.cuda.OutOfMemoryError):

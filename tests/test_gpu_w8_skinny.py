@@ -1,4 +1,5 @@
-"""W8A16 for few rows of A: column strips with K split over workgroups.
+"""W8A16 for few rows of A, for unaligned operands, and with K split over
+workgroups.
 
 Against the float64 oracle on the fp16 activations.  Products of f16 and int8
 are exact in f32 and every sum is f32, so an element is within
@@ -111,3 +112,44 @@ def test_graph_replays(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(c, eager)
+
+
+# Every boundary of the unaligned 128 x 128-tile kernel: odd K, N and row
+# strides, bases of A on 2 bytes and of B on any byte, single elements, K one
+# short of and one past a step, ragged tiles in both directions; NaN in every
+# element of A outside its rows.
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("m,n,k,lda,ldb,da,db", [
+    (1, 1, 1, 1, 1, 0, 0), (1, 1, 1, 3, 5, 1, 3), (3, 7, 63, 64, 8, 0, 1), (5, 130, 65, 65, 131, 1, 2),
+    (128, 128, 64, 65, 129, 0, 0), (129, 127, 127, 127, 127, 1, 1), (70, 256, 129, 136, 256, 4, 5),
+    (200, 257, 640, 641, 259, 3, 3), (65, 301, 1999, 2001, 301, 0, 2)])
+def test_unaligned(gpu, m, n, k, lda, ldb, da, db, scaled):
+    a, b, s = _inputs(m, n, k, m + n + k, lda=lda, ldb=ldb)
+    a[:, k:] = float("nan")
+    abuf = torch.full((da + m * lda + 8,), float("nan"), dtype=torch.float16)
+    abuf[da:da + m * lda] = a.reshape(-1)
+    bbuf = torch.full((db + k * ldb,), 77, dtype=torch.int8)
+    bbuf[db:] = b.reshape(-1)
+    c = torch.full((m, n + 3), 5.0, device=DEV)
+    ad, bd = abuf.to(DEV)[da:], bbuf.to(DEV)[db:]
+    if scaled:
+        neso_amd.w8a16_scaled_matmul(ad, bd, c, s.to(DEV), k, lda, ldb, n + 3, M=m, N=n)
+    else:
+        neso_amd.w8a16_matmul(ad, bd, c, k, lda, ldb, n + 3, M=m, N=n)
+    c = c.cpu()
+    assert Q.rel_err(c[:, :n].numpy(), _ref(a, b, s if scaled else None, k, n)) < 1e-5
+    assert torch.all(c[:, n:] == 5.0)
+
+
+# Split tiles: the last range short, more ranges than steps allow, and a
+# result whose rows are no multiple of four.
+@pytest.mark.parametrize("m,n,k", [(128, 1024, 1032), (100, 304, 4000), (300, 501, 2001), (65, 128, 8192)])
+def test_split_tiles(gpu, m, n, k):
+    a, b, s = _inputs(m, n, k, m + n + k)
+    ad, bd, sd = a.to(DEV), b.to(DEV), s.to(DEV)
+    c = torch.full((m, n), float("nan"), device=DEV)
+    plan = neso_amd.launch_plan("w8a16_scaled_matmul", ad, bd, c, sd, k, k, n, n, M=m, N=n, cu_count=256)
+    assert [p["device_kernel"] for p in plan] == ["w8a16_gemm_kernel", "w8a16_reduce_kernel"]
+    assert plan[0]["grid"][2] > 1
+    neso_amd.w8a16_scaled_matmul(ad, bd, c, sd, k, k, n, n, M=m, N=n)
+    assert Q.rel_err(c.cpu().numpy(), _ref(a, b, s, k, n)) < 1e-5
