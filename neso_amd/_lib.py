@@ -110,6 +110,8 @@ class NesoArgumentError(NesoError, ValueError):
 def load() -> ctypes.CDLL:
     """Load the library once; raise if it is missing or incomplete."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

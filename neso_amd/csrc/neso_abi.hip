@@ -44,7 +44,7 @@ bool aligned2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0
 // Optional override of the FA2 key split, for tuning and for tests that
 // exercise every code path: NESO_AMD_FA2_KSPLIT=1..4.
 int env_ksplit() {
-  const char* v = getenv("NESO_AMD_FA2_KSPLIT");
+  const char* v = neso::tuning_env("NESO_AMD_FA2_KSPLIT");
   if (!v) return 0;
   const int k = atoi(v);
   return (k >= 1 && k <= 4) ? k : 0;
@@ -55,7 +55,7 @@ int env_ksplit() {
 // generic kernel, =2 the fast kernel wherever it applies; unset or 1
 // chooses by shape.
 int env_allow_fast() {
-  const char* v = getenv("NESO_AMD_FA2_FAST");
+  const char* v = neso::tuning_env("NESO_AMD_FA2_FAST");
   if (!v) return 1;
   if (v[0] == '0') return 0;
   return v[0] == '2' ? 2 : 1;
@@ -64,7 +64,7 @@ int env_allow_fast() {
 // Query waves per key group of either FA2 kernel (tests cover both):
 // NESO_AMD_FA2_QW=2 or 4; unset chooses from the grid size.
 int env_qwaves() {
-  const char* v = getenv("NESO_AMD_FA2_QW");
+  const char* v = neso::tuning_env("NESO_AMD_FA2_QW");
   if (!v) return 0;
   const int k = atoi(v);
   return (k == 2 || k == 4) ? k : 0;
@@ -74,7 +74,7 @@ int env_qwaves() {
 // paired 128-row query blocks, 2 forces paired 64-row halves (no window
 // only), 0 forbids both; unset lets the launcher choose.
 int env_pair() {
-  const char* v = getenv("NESO_AMD_FA2_PAIR");
+  const char* v = neso::tuning_env("NESO_AMD_FA2_PAIR");
   if (!v) return -1;
   const int k = atoi(v);
   return (k == 1 || k == 2) ? k : 0;
@@ -165,7 +165,15 @@ thread_local PlanState g_plan;
 
 }  // namespace
 
+extern char** environ;
+
 namespace neso {
+
+const char* tuning_env(const char* name) {
+  for (char** e = environ; e && *e; ++e)
+    if ((*e)[0] == 'N' && strncmp(*e, "NESO_AMD_", 9) == 0) return getenv(name);
+  return nullptr;
+}
 
 bool plan_recording() { return g_plan.active; }
 

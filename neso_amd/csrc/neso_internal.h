@@ -53,6 +53,10 @@ struct Fa2Args {
 // launch-plan recording stands in for.
 int device_cu_count();
 
+// getenv for the NESO_AMD_* tuning variables: one short scan of the
+// environment when none is set, the usual case, instead of one per variable.
+const char* tuning_env(const char* name);
+
 // ---- launches ----
 // Every kernel of the library is launched through launch<&kernel>(...).
 // While a launch plan is being recorded on the calling thread

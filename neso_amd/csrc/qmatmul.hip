@@ -1250,7 +1250,7 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   // overrides the largest GEMV M.
   // Values outside 0..4 fall back to the default: the GEMV kernels hold
   // at most four rows of X.
-  const char* gemv_env = getenv("NESO_AMD_W4_GEMV_MAX_M");
+  const char* gemv_env = tuning_env("NESO_AMD_W4_GEMV_MAX_M");
   const int gemv_env_m = gemv_env ? atoi(gemv_env) : -1;
   const int gemv_max_m = (gemv_env_m >= 0 && gemv_env_m <= 4) ? gemv_env_m : 2;
   // Up to K = 16384 the GEMV also serves M = 1, and M = 2 while N leaves two
@@ -1306,9 +1306,9 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   // 64 x 64 with four; 6: 32 x 64 with four; 7: 32 x 32 with eight.
   // NESO_AMD_W4_WIDE_TILE_MIN_M (65 by default) is the smallest M for which
   // those 128 x 128 tiles are taken when no fine tile fits.
-  const char* tile_env = getenv("NESO_AMD_W4_TILE_GEMM");
+  const char* tile_env = tuning_env("NESO_AMD_W4_TILE_GEMM");
   const int tile_mode = tile_env ? atoi(tile_env) : -1;
-  const char* wide_env = getenv("NESO_AMD_W4_WIDE_TILE_MIN_M");
+  const char* wide_env = tuning_env("NESO_AMD_W4_WIDE_TILE_MIN_M");
   const int wide_min_m = wide_env ? atoi(wide_env) : 65;
   const int cus = device_cu_count();
   auto tiles_of = [&](int tm, int tn) { return ((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn); };
@@ -1330,7 +1330,7 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
   // the 32 x 32 tile grid would not fit on the CUs), and up to M = 32 when
   // the tile GEMM is off or its offsets would pass 2^31 bytes.
   // NESO_AMD_W4_SKINNY_MAX_M (at most 64) forces them up to that M.
-  const char* skinny_env = getenv("NESO_AMD_W4_SKINNY_MAX_M");
+  const char* skinny_env = tuning_env("NESO_AMD_W4_SKINNY_MAX_M");
   const int skinny_max_m = skinny_env ? atoi(skinny_env) : 32;
   // Up to M = 16 past the X-in-LDS kernel's K the 32 x 32 tile GEMM beats
   // the split-K skinny kernel when its grid fits (K = 11008 N = 4096:
@@ -1395,7 +1395,7 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
     // form's one-wave groups take neither).
     static constexpr int kGroups[8] = {0, 1, 2, 2, 4, 4, 4, 8}, kRowTiles[8] = {0, 4, 4, 4, 4, 2, 1, 1};
     const int kgroups = kGroups[mode], steps = ((a.K + kTK - 1) / kTK + kgroups - 1) / kgroups;
-    const char* sync_env = getenv("NESO_AMD_W4_TILE_SYNC");
+    const char* sync_env = tuning_env("NESO_AMD_W4_TILE_SYNC");
     W4Args t = a;
     t.group_sync = kgroups > 1 && (sync_env ? atoi(sync_env) != 0
                                             : steps >= (kRowTiles[mode] == 4 ? 16 : 32));

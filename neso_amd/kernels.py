@@ -49,19 +49,19 @@ __all__ = [
 
 def _ptr(x: Any, name: str, dtype: torch.dtype | tuple[torch.dtype, ...] | None) -> int:
     """Device address of a tensor (dtype/device checked) or a raw integer address."""
+    if isinstance(x, torch.Tensor):
+        if not x.is_cuda:
+            raise ValueError(f"{name}: tensor must be on the GPU (got {x.device}); there is no CPU path")
+        if x.dtype is not dtype and dtype is not None:
+            allowed = dtype if isinstance(dtype, tuple) else (dtype,)
+            if x.dtype not in allowed:
+                raise TypeError(f"{name}: dtype {x.dtype} not in {allowed}")
+        return x.data_ptr()
     if x is None:
         return 0
     if isinstance(x, int):
         return x
-    if not isinstance(x, torch.Tensor):
-        raise TypeError(f"{name}: expected a torch.Tensor or a device address, got {type(x)!r}")
-    if x.device.type != "cuda":
-        raise ValueError(f"{name}: tensor must be on the GPU (got {x.device}); there is no CPU path")
-    if dtype is not None:
-        allowed = dtype if isinstance(dtype, tuple) else (dtype,)
-        if x.dtype not in allowed:
-            raise TypeError(f"{name}: dtype {x.dtype} not in {allowed}")
-    return x.data_ptr()
+    raise TypeError(f"{name}: expected a torch.Tensor or a device address, got {type(x)!r}")
 
 
 def _extent(x: Any, name: str, elems: int) -> None:
@@ -72,7 +72,7 @@ def _extent(x: Any, name: str, elems: int) -> None:
     so a short tensor would be read or written past its allocation.  Raw
     integer addresses are the caller's responsibility.
     """
-    if not isinstance(x, torch.Tensor) or elems <= 0:
+    if not isinstance(x, torch.Tensor) or elems <= 0 or (elems <= x.numel() and x.is_contiguous()):
         return
     avail = x.untyped_storage().nbytes() - x.storage_offset() * x.element_size()
     if elems * x.element_size() > avail:
@@ -80,25 +80,31 @@ def _extent(x: Any, name: str, elems: int) -> None:
                          f"tensor holds {avail // x.element_size()} from its first element")
 
 
-def _require(cond: bool, msg: str) -> None:
-    if not cond:
-        raise ValueError(msg)
+_F16_F32 = (torch.float16, torch.float32)
 
 
 def _stream(stream: Any, *tensors: Any) -> int:
     if stream is not None:
         return int(stream.cuda_stream) if hasattr(stream, "cuda_stream") else int(stream)
     for t in tensors:
-        if isinstance(t, torch.Tensor) and t.device.type == "cuda":
-            return int(torch.cuda.current_stream(t.device).cuda_stream)
+        if isinstance(t, torch.Tensor) and t.is_cuda:
+            return _current_stream(t.get_device())
     return 0
+
+
+# The handle of torch.cuda.current_stream(device), without the Stream object.
+_current_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") \
+    else lambda index: int(torch.cuda.current_stream(index).cuda_stream)
+
+
+_NO_CONTEXT = contextlib.nullcontext()
 
 
 def _on_stream(stream: int, device):
     """Context that makes ``stream`` (a raw HIP stream handle) torch's current
     stream, so that torch work in it is ordered with the launch."""
-    if torch.cuda.current_stream(device).cuda_stream == stream:
-        return contextlib.nullcontext()
+    if _current_stream(device.index) == stream:
+        return _NO_CONTEXT
     return torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device))
 
 
@@ -297,14 +303,6 @@ def flash_attention_fwd(Q, K, V, O, N: int, stride_qo: int, stride_kv: int, scal
     (V), so any finite magnitude keeps fp32-class accuracy.  Without it, or
     under graph capture, fp32 elements must lie below 65504 in magnitude.
     """
-    _flash_attention_fwd(Q, K, V, O, N, stride_qo, stride_kv, scale, head_dim, batch_heads,
-                         stride_bh_qo, stride_bh_kv, causal, qkv_dtype, check_range, stream, False)
-
-
-def _flash_attention_fwd(Q, K, V, O, N, stride_qo, stride_kv, scale, head_dim, batch_heads,
-                         stride_bh_qo, stride_bh_kv, causal, qkv_dtype, check_range, stream,
-                         own_out: bool) -> None:
-    """flash_attention_fwd; ``own_out`` as in _checked_launch."""
     if head_dim is None:
         if not isinstance(Q, torch.Tensor):
             raise ValueError("head_dim is required when Q is a raw address")
@@ -319,19 +317,31 @@ def _flash_attention_fwd(Q, K, V, O, N, stride_qo, stride_kv, scale, head_dim, b
         for t, nm, sp in ((Q, "Q", span_q), (K, "K", span_kv), (V, "V", span_kv),
                           (O, "O", span_q)):
             _extent(t, nm, sp)
-    dt = torch.float32 if qkv_dtype == "f32" else torch.float16
+    _launch_fa2(Q, K, V, O, int(N), int(stride_qo), int(stride_kv), float(scale), int(head_dim),
+                int(batch_heads), int(stride_bh_qo), int(stride_bh_kv), int(bool(causal)),
+                qkv_dtype == "f32", check_range, _stream(stream, Q, O), False)
+
+
+def _launch_fa2(Q, K, V, O, N, stride_qo, stride_kv, scale, head_dim, batch_heads, stride_bh_qo,
+                stride_bh_kv, causal, f32, check_range, st, own_out) -> None:
+    """The FA2 call once its extents are checked."""
     lib = _lib.load()
-    fn = lib.neso_flash_attention_f32_fwd if qkv_dtype == "f32" else lib.neso_flash_attention_fwd
-    st = _stream(stream, Q, O)
+    if not f32:
+        f16 = torch.float16
+        status = lib.neso_flash_attention_fwd(
+            _ptr(Q, "Q", f16), _ptr(K, "K", f16), _ptr(V, "V", f16), _ptr(O, "O", torch.float32), N,
+            stride_qo, stride_kv, scale, head_dim, batch_heads, stride_bh_qo, stride_bh_kv, causal, st)
+        if status:
+            _lib.check(status)
+        return
+    dt = torch.float32
 
     def launch_kernel(Q, K, V, scale):
-        _lib.check(fn(
-            _ptr(Q, "Q", dt), _ptr(K, "K", dt), _ptr(V, "V", dt),
-            _ptr(O, "O", torch.float32), int(N), int(stride_qo), int(stride_kv), float(scale),
-            int(head_dim), int(batch_heads), int(stride_bh_qo), int(stride_bh_kv),
-            int(bool(causal)), st))
+        _lib.check(lib.neso_flash_attention_f32_fwd(
+            _ptr(Q, "Q", dt), _ptr(K, "K", dt), _ptr(V, "V", dt), _ptr(O, "O", dt), N, stride_qo,
+            stride_kv, scale, head_dim, batch_heads, stride_bh_qo, stride_bh_kv, causal, st))
 
-    if qkv_dtype == "f32" and check_range and N > 0 and batch_heads > 0:
+    if check_range and N > 0 and batch_heads > 0:
         _checked_launch(
             launch_kernel, Q, K, V, O, scale,
             [(t, nm, (batch_heads, N, head_dim), (sb, sr, 1))
@@ -414,13 +424,19 @@ def flash_attention_window_fwd(Q, K, V, O, seq_len: int, stride_h: int, stride_m
         span = (seq_len - 1) * stride_m + (num_heads - 1) * stride_h + head_dim
         for t, nm in ((Q, "Q"), (K, "K"), (V, "V"), (O, "O")):
             _extent(t, nm, span)
-    lib = _lib.load()
-    st = lib.neso_flash_attention_window_fwd(
-        _ptr(Q, "Q", torch.float16), _ptr(K, "K", torch.float16), _ptr(V, "V", torch.float16),
-        _ptr(O, "O", (torch.float16, torch.float32)), int(seq_len), int(stride_h), int(stride_m),
-        float(sm_scale), int(window_left), int(window_right), int(num_heads), int(head_dim),
-        int(out_dtype), _stream(stream, Q, O))
-    _lib.check(st)
+    _launch_window(Q, K, V, O, int(seq_len), int(stride_h), int(stride_m), float(sm_scale),
+                   int(window_left), int(window_right), int(num_heads), int(head_dim), out_dtype,
+                   _stream(stream, Q, O))
+
+
+def _launch_window(Q, K, V, O, seq_len, stride_h, stride_m, sm_scale, window_left, window_right,
+                   num_heads, head_dim, out_dtype, st) -> None:
+    f16 = torch.float16
+    status = _lib.load().neso_flash_attention_window_fwd(
+        _ptr(Q, "Q", f16), _ptr(K, "K", f16), _ptr(V, "V", f16), _ptr(O, "O", _F16_F32), seq_len,
+        stride_h, stride_m, sm_scale, window_left, window_right, num_heads, head_dim, out_dtype, st)
+    if status:
+        _lib.check(status)
 
 
 def rel_pos_fa2_fwd(Q, K, V, bias, O, T: int, stride: int, scale: float, stride_h: int,
@@ -451,13 +467,20 @@ def rel_pos_fa2_fwd(Q, K, V, bias, O, T: int, stride: int, scale: float, stride_
             _extent(t, nm, span)
         per_head = T * T if bias_mode == _lib.NESO_BIAS_DENSE_SCALED_F16 else 2 * T - 1
         _extent(bias, "bias", (num_heads - 1) * bias_stride_h + per_head)
-    lib = _lib.load()
-    st = lib.neso_rel_pos_fa2_fwd(
-        _ptr(Q, "Q", torch.float16), _ptr(K, "K", torch.float16), _ptr(V, "V", torch.float16),
-        _ptr(bias, "bias", bias_dtype), _ptr(O, "O", (torch.float16, torch.float32)), int(T),
-        int(stride), float(scale), int(stride_h), int(bias_stride_h), int(num_heads),
-        int(head_dim), int(bias_mode), int(out_dtype), _stream(stream, Q, O))
-    _lib.check(st)
+    _launch_rel_pos(Q, K, V, bias, O, int(T), int(stride), float(scale), int(stride_h),
+                    int(bias_stride_h), int(num_heads), int(head_dim), int(bias_mode), bias_dtype,
+                    out_dtype, _stream(stream, Q, O))
+
+
+def _launch_rel_pos(Q, K, V, bias, O, T, stride, scale, stride_h, bias_stride_h, num_heads, head_dim,
+                    bias_mode, bias_dtype, out_dtype, st) -> None:
+    f16 = torch.float16
+    status = _lib.load().neso_rel_pos_fa2_fwd(
+        _ptr(Q, "Q", f16), _ptr(K, "K", f16), _ptr(V, "V", f16), _ptr(bias, "bias", bias_dtype),
+        _ptr(O, "O", _F16_F32), T, stride, scale, stride_h, bias_stride_h, num_heads, head_dim,
+        bias_mode, out_dtype, st)
+    if status:
+        _lib.check(status)
 
 
 def rel_pos_precompute(Q, K_rel, bias_u, bias_v, T: int, d: int, nh: int, scale: float, Q_u,
@@ -540,12 +563,17 @@ def w4a16_matmul(X, W, scales, Y, M: int, N: int, K: int, stride_xm: int, stride
         _extent(W, "W", N * (K // 8))
         _extent(scales, "scales", N * (K // group_size))
         _extent(Y, "Y", (M - 1) * stride_ym + N)
-    lib = _lib.load()
-    st = lib.neso_w4a16_matmul(
-        _ptr(X, "X", torch.float16), _ptr(W, "W", torch.int32), _ptr(scales, "scales", torch.float16),
-        _ptr(Y, "Y", torch.float16), int(M), int(N), int(K), int(stride_xm), int(stride_ym),
-        int(group_size), int(zero_point), _stream(stream, X, Y))
-    _lib.check(st)
+    _launch_w4(X, W, scales, Y, int(M), int(N), int(K), int(stride_xm), int(stride_ym),
+               int(group_size), int(zero_point), _stream(stream, X, Y))
+
+
+def _launch_w4(X, W, scales, Y, M, N, K, stride_xm, stride_ym, group_size, zero_point, st) -> None:
+    f16 = torch.float16
+    status = _lib.load().neso_w4a16_matmul(
+        _ptr(X, "X", f16), _ptr(W, "W", torch.int32), _ptr(scales, "scales", f16), _ptr(Y, "Y", f16), M,
+        N, K, stride_xm, stride_ym, group_size, zero_point, st)
+    if status:
+        _lib.check(status)
 
 
 def _w8_extents(A, B, C, scale, K, stride_am, stride_bk, stride_cm, M, N) -> None:
@@ -667,11 +695,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
     own_out = out is None
     if own_out:
         out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-    _require(out.shape == q.shape and out.is_contiguous() and out.dtype == torch.float32,
-             f"out must be a contiguous fp32 tensor of shape {tuple(q.shape)}")
+    elif out.shape != q.shape or not out.is_contiguous() or out.dtype != torch.float32:
+        raise ValueError(f"out must be a contiguous fp32 tensor of shape {tuple(q.shape)}")
     scale = 1.0 / math.sqrt(d) if scale is None else scale
-    _flash_attention_fwd(q, k, v, out, n, d, d, scale, d, bh, n * d, n * d, causal, None,
-                         check_range, None, own_out)
+    # Contiguous tensors of one shape: every declared extent holds.
+    _launch_fa2(q, k, v, out, n, d, d, float(scale), d, bh, n * d, n * d, int(bool(causal)),
+                q.dtype == torch.float32, check_range, _stream(None, q, out), own_out)
     return out
 
 
@@ -679,26 +708,30 @@ def rel_pos_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, table: 
                       scale: float | None = None, out_dtype: torch.dtype = torch.float32,
                       out: torch.Tensor | None = None) -> torch.Tensor:
     """softmax(Q K^T * scale + table[h, i - j + N - 1]) V for [H, N, d] fp16, table f32 [H, 2N-1]."""
-    _require(q.dim() == 3, f"q must be [H, N, d], got {tuple(q.shape)}")
-    _require(k.shape == q.shape and v.shape == q.shape,
-             f"k {tuple(k.shape)} and v {tuple(v.shape)} must match q {tuple(q.shape)}")
-    _require(q.is_contiguous() and k.is_contiguous() and v.is_contiguous(),
-             "q, k, v must be contiguous")
-    _require(q.dtype == k.dtype == v.dtype == torch.float16, "q, k, v must be fp16")
+    if q.dim() != 3:
+        raise ValueError(f"q must be [H, N, d], got {tuple(q.shape)}")
+    if k.shape != q.shape or v.shape != q.shape:
+        raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} must match q {tuple(q.shape)}")
+    if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
+        raise ValueError("q, k, v must be contiguous")
+    if not q.dtype == k.dtype == v.dtype == torch.float16:
+        raise ValueError("q, k, v must be fp16")
     h, n, d = (int(s) for s in q.shape)
     if table.shape != (h, 2 * n - 1):
         raise ValueError(f"table must be [H, 2N-1] = [{h}, {2 * n - 1}], got {tuple(table.shape)}")
-    _require(table.is_contiguous() and table.dtype == torch.float32,
-             "table must be a contiguous fp32 tensor")
-    _require(out_dtype in (torch.float16, torch.float32), "out_dtype must be fp16 or fp32")
-    if out is not None:
-        _require(out.shape == q.shape and out.is_contiguous() and out.dtype == out_dtype,
-                 f"out must be a contiguous {out_dtype} tensor of shape {tuple(q.shape)}")
+    if not table.is_contiguous() or table.dtype != torch.float32:
+        raise ValueError("table must be a contiguous fp32 tensor")
+    if out_dtype not in _F16_F32:
+        raise ValueError("out_dtype must be fp16 or fp32")
     if out is None:
         out = torch.empty((h, n, d), dtype=out_dtype, device=q.device)
+    elif out.shape != q.shape or not out.is_contiguous() or out.dtype != out_dtype:
+        raise ValueError(f"out must be a contiguous {out_dtype} tensor of shape {tuple(q.shape)}")
     scale = 1.0 / math.sqrt(d) if scale is None else scale
-    rel_pos_fa2_fwd(q, k, v, table, out, n, d, scale, n * d, 2 * n - 1, num_heads=h, head_dim=d,
-                    bias_mode=_lib.NESO_BIAS_TABLE_F32)
+    _launch_rel_pos(q, k, v, table, out, n, d, float(scale), n * d, 2 * n - 1, h, d,
+                    _lib.NESO_BIAS_TABLE_F32, torch.float32,
+                    _lib.NESO_OUT_F32 if out_dtype == torch.float32 else _lib.NESO_OUT_F16,
+                    _stream(None, q, out))
     return out
 
 
@@ -708,14 +741,17 @@ def precompute_bias_and_qu(q: torch.Tensor, k_rel: torch.Tensor, bias_u: torch.T
     (tests/test_rel_pos_fa2.py:286-311) on fp32 tensors q [nh, T, d],
     k_rel [nh, 2T-1, d], bias_u / bias_v [nh, d]; returns (Q_u fp16
     [nh, T, d], rel_bias fp16 [nh, T, T]) for :func:`rel_pos_fa2_fwd`."""
-    _require(q.dim() == 3, f"q must be [nh, T, d], got {tuple(q.shape)}")
+    if q.dim() != 3:
+        raise ValueError(f"q must be [nh, T, d], got {tuple(q.shape)}")
     nh, t, d = (int(x) for x in q.shape)
-    _require(tuple(k_rel.shape) == (nh, 2 * t - 1, d),
-             f"k_rel must be [nh, 2T-1, d] = [{nh}, {2 * t - 1}, {d}], got {tuple(k_rel.shape)}")
+    if k_rel.shape != (nh, 2 * t - 1, d):
+        raise ValueError(f"k_rel must be [nh, 2T-1, d] = [{nh}, {2 * t - 1}, {d}], got {tuple(k_rel.shape)}")
     for x, nm in ((bias_u, "bias_u"), (bias_v, "bias_v")):
-        _require(tuple(x.shape) == (nh, d), f"{nm} must be [nh, d] = [{nh}, {d}]")
+        if x.shape != (nh, d):
+            raise ValueError(f"{nm} must be [nh, d] = [{nh}, {d}]")
     for x, nm in ((q, "q"), (k_rel, "k_rel"), (bias_u, "bias_u"), (bias_v, "bias_v")):
-        _require(x.is_contiguous() and x.dtype == torch.float32, f"{nm} must be contiguous fp32")
+        if not x.is_contiguous() or x.dtype != torch.float32:
+            raise ValueError(f"{nm} must be contiguous fp32")
     q_u = torch.empty((nh, t, d), dtype=torch.float16, device=q.device)
     rel_bias = torch.empty((nh, t, t), dtype=torch.float16, device=q.device)
     _rel_pos_precompute(q, k_rel, bias_u, bias_v, t, d, nh, 1.0 / math.sqrt(d), q_u, rel_bias, True, None,
@@ -736,12 +772,12 @@ def window_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window_l
     n, h, d = (int(x) for x in q.shape)
     if out is None:
         out = torch.empty((n, h, d), dtype=out_dtype, device=q.device)
-    _require(out.shape == q.shape and out.is_contiguous()
-             and out.dtype in (torch.float16, torch.float32),
-             f"out must be a contiguous fp16 or fp32 tensor of shape {tuple(q.shape)}")
+    if out.shape != q.shape or not out.is_contiguous() or out.dtype not in _F16_F32:
+        raise ValueError(f"out must be a contiguous fp16 or fp32 tensor of shape {tuple(q.shape)}")
     scale = 1.0 / math.sqrt(d) if scale is None else scale
-    flash_attention_window_fwd(q, k, v, out, n, d, h * d, scale, window_left, window_right,
-                               num_heads=h, head_dim=d)
+    _launch_window(q, k, v, out, n, d, h * d, float(scale), int(window_left), int(window_right), h, d,
+                   _lib.NESO_OUT_F32 if out.dtype == torch.float32 else _lib.NESO_OUT_F16,
+                   _stream(None, q, out))
     return out
 
 
@@ -749,25 +785,24 @@ def w4a16_linear(x: torch.Tensor, w_packed: torch.Tensor, scales: torch.Tensor, 
                  group_size: int = 32, zero_point: int = 8,
                  out: torch.Tensor | None = None) -> torch.Tensor:
     """x [M, K] fp16 @ dequant(w_packed [N, K/8] int32, scales [N, K/group])^T -> fp16 [M, N]."""
-    _require(x.dim() == 2 and x.stride(1) == 1, "x must be [M, K] with unit column stride")
+    if x.dim() != 2 or x.stride(1) != 1:
+        raise ValueError("x must be [M, K] with unit column stride")
     m, k = (int(s) for s in x.shape)
-    _require(w_packed.dim() == 2 and w_packed.is_contiguous() and w_packed.dtype == torch.int32,
-             "w_packed must be a contiguous int32 [N, K/8] tensor")
+    if w_packed.dim() != 2 or not w_packed.is_contiguous() or w_packed.dtype != torch.int32:
+        raise ValueError("w_packed must be a contiguous int32 [N, K/8] tensor")
     n = int(w_packed.shape[0])
-    _require(k % 8 == 0 and int(w_packed.shape[1]) == k // 8,
-             f"w_packed must be [N, K/8] = [{n}, {k // 8}], got {tuple(w_packed.shape)}")
-    _require(group_size > 0 and k % group_size == 0,
-             f"group_size {group_size} must divide K = {k}")
-    _require(scales.dim() == 2 and scales.is_contiguous() and scales.dtype == torch.float16
-             and tuple(scales.shape) == (n, k // group_size),
-             f"scales must be a contiguous fp16 [N, K/group] = [{n}, {k // group_size}] tensor, "
-             f"got {tuple(scales.shape)} {scales.dtype}")
-    if out is not None:
-        _require(out.dim() == 2 and tuple(out.shape) == (m, n) and out.stride(1) == 1
-                 and out.dtype == torch.float16,
-                 f"out must be fp16 [M, N] = [{m}, {n}] with unit column stride")
+    if k % 8 != 0 or int(w_packed.shape[1]) != k // 8:
+        raise ValueError(f"w_packed must be [N, K/8] = [{n}, {k // 8}], got {tuple(w_packed.shape)}")
+    if group_size <= 0 or k % group_size != 0:
+        raise ValueError(f"group_size {group_size} must divide K = {k}")
+    if scales.dim() != 2 or not scales.is_contiguous() or scales.dtype != torch.float16 \
+            or scales.shape != (n, k // group_size):
+        raise ValueError(f"scales must be a contiguous fp16 [N, K/group] = [{n}, {k // group_size}] tensor, "
+                         f"got {tuple(scales.shape)} {scales.dtype}")
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=x.device)
-    w4a16_matmul(x, w_packed, scales, out, m, n, k, x.stride(0), out.stride(0), group_size,
-                 zero_point)
+    elif out.dim() != 2 or out.shape != (m, n) or out.stride(1) != 1 or out.dtype != torch.float16:
+        raise ValueError(f"out must be fp16 [M, N] = [{m}, {n}] with unit column stride")
+    _launch_w4(x, w_packed, scales, out, m, n, k, x.stride(0), out.stride(0), int(group_size),
+               int(zero_point), _stream(None, x, out))
     return out
