@@ -566,8 +566,10 @@ __global__ __launch_bounds__(WM * WN * kWave) void w4a16_gemm_kernel(W4Args a) {
 // 32 w .. 32 w + 31 of the tile for all its rows (MI x 1
 // v_mfma_f32_32x32x16_f16 tiles), so no two waves of a group need the same
 // weights and each code is dequantised once per workgroup:
-//   * W: lane (n = l%32, h = l/32) loads word quad h (32 codes, 16 bytes,
-//     one scale group) of its row's step and its scale, and dequantises
+//   * W: lane (n = l%32, h = l/32) takes word quad h (32 codes, 16 bytes,
+//     one scale group) of its row's step and its scale (staged packed through
+//     LDS four steps at a time, or straight from memory for groups that are
+//     no power of two), and dequantises
 //     (c - z) * s (one fp16 rounding) straight into MFMA B operands: MFMA
 //     ks of the step takes word ks, i.e. codes 32 h + 8 ks + {0,4,1,5,2,6,
 //     3,7}, the order of unpack_word_x16;
@@ -577,19 +579,21 @@ __global__ __launch_bounds__(WM * WN * kWave) void w4a16_gemm_kernel(W4Args a) {
 //     t/8 + 8 WN j.  A wave's A fragment for MFMA (mi, ks) is row
 //     32 mi + l%32 at codes 32 h + 8 ks of the step, one ds_read_b128.
 // Per step and wave: 4 MI MFMAs, 4 MI fragment reads, 4 dequantised words
-// and 4 MI / WN X stores.  Only X is stored to LDS; that store stream (LDS
-// writes run at about a third of the read rate on gfx950) was the cost of
-// the earlier form, which dequantised W into LDS too.  LDS is
-// double-buffered per group; X loads run two steps ahead of their store, W
-// loads two steps ahead of their use; the next step's X stores are issued
-// among the current step's MFMAs.  One sync per step: a workgroup barrier,
+// and 4 MI / WN X stores (and one packed 16-byte W store and read).  The LDS
+// store stream (LDS writes run at about a third of the read rate on gfx950)
+// was the cost of the earlier form, which dequantised W into LDS.  X is
+// double-buffered per group; its loads run two steps ahead of their store,
+// W loads four to eight steps ahead of their use (two when not staged); the
+// next step's X stores are issued among the current step's MFMAs.  One sync per step: a workgroup barrier,
 // a per-group LDS arrival counter, or for one-wave groups a wave-level
 // fence (step_sync below).
 constexpr int kTT = 128, kTK = 64, kTLD = kTK + 8;
 
 // K-groups per workgroup, waves (32-column strips) per group, 32-row MFMA
 // tiles per wave (tile rows 32 MI).
-template <int kTKG, int WN = 4, int MI = 4>
+// GS: scales per four steps (256 codes) with W staged through LDS, 8, 4 or 2
+// for groups of 32, 64, and 128 or more; 0: W straight from memory.
+template <int kTKG, int WN, int MI, int GS>
 __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args a) {
   static_assert(WN == 1 || WN == 2 || WN == 4, "waves per group");
   static_assert(MI == 1 || MI == 2 || MI == 4, "32-row tiles per wave");
@@ -603,6 +607,7 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
   static_assert(XP >= 1 && XP * GT == TM * 8, "X pieces");
   __shared__ half8v lds[kTKG][2][kBuf];   // [group][buffer] X tile
   __shared__ uint32_t arrivals[kTKG];      // per-group arrival counters
+  __shared__ uint4v wlds[GS ? kTKG * WN : 1][GS ? 256 : 1];  // [wave] four steps of 32 rows of W
   const int tid = threadIdx.x % GT, lane = tid & 63;
   const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -624,7 +629,9 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
   const uint32_t gshift = __builtin_ctz(gm);
   // Steps per group (every group runs the same count, as the workgroup
   // barriers require); steps past K read zeros.
-  const int T = ((a.K + kTK - 1) / kTK + kTKG - 1) / kTKG;
+  // Staged W takes an even count, so that ranges start at multiples of 128.
+  const int T0 = ((a.K + kTK - 1) / kTK + kTKG - 1) / kTKG;
+  const int T = GS ? (T0 + 1) & ~1 : T0;
 
   // X: row tid/8 + 8 WN j, 16-byte piece tid%8 of the step.  W: row
   // 32 wave + li of the tile, word quad lh of the step.
@@ -639,7 +646,7 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
   };
   auto xload = [&](XStage& g, int t) {
     const int k = (kg * T + t) * kTK + 8 * xp;
-    const uint32_t xoob = k < a.K ? 0u : kOut;
+    const uint32_t xoob = (!GS || t < T) && k < a.K ? 0u : kOut;
 #pragma unroll
     for (int j = 0; j < XP; ++j)
       g.x[j] = buf_load_half8(rx, (((uint32_t)(xr0 + 8 * WN * j) * a.ldx + k) * 2u) | xoob);
@@ -652,6 +659,65 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
                                          rw, ((uint32_t)wrow * KW * 4u + chunk * 16u) | woob, 0, 0));
     g.s = __builtin_bit_cast(half_t, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
                                          rs, (((uint32_t)wrow * SG + sidx) * 2u) | woob, 0, 0));
+  };
+  // Staged W, four steps (128 bytes of each row) at a time: eight lanes read
+  // a row's line, eight rows per instruction, and the wave's 4 KiB go through
+  // its own part of LDS to the lanes that use them, piece p of row r at
+  // p ^ (r / 2) % 8 (write passes of one row and read passes of 16 rows at
+  // one piece both spread over all banks).  Read per step instead, lane
+  // (n, h) its own 16 bytes, every lane is an L1 access of its own: 64 for
+  // 1 KiB where 16 suffice, and the L1's access rate was at 65-70% of its
+  // limit (TCP_TOTAL_CACHE_ACCESSES, M = 256).  The scales of the four steps
+  // come with them, one load per lane.  us before / now: K 4096 N 4096 M 64
+  // 12.2 / 10.3, M 256 20.0 / 18.4, M 1024 47.5 / 44.3; N 11008 M 256 39.9 /
+  // 37.9, M 2048 241 / 226; K 11008 N 4096 M 64 26.4 / 21.5, M 128 37.7 /
+  // 30.7, M 256 49.5 / 43.3.  X loads four steps ahead instead of two: equal
+  // or up to 6% slower.
+  typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+  struct WBatch {
+    uint4v w[4];
+    uint4v s;
+  };
+  uint4v* const wl = wlds[GS ? kg * WN + wave : 0];
+  const int wr8 = lane >> 3, wp8 = lane & 7;
+  auto bload = [&](WBatch& b, int t) {
+    const uint32_t step0 = (uint32_t)(kg * T + t);
+    const uint32_t oob = t < T && (int)(step0 * kTK) < a.K ? 0u : kOut;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      b.w[i] = __builtin_bit_cast(
+          uint4v, __builtin_amdgcn_raw_buffer_load_b128(
+                      rw, ((uint32_t)(32 * wave + 8 * i + wr8) * KW * 4u + step0 * 32u + wp8 * 16u) | oob, 0, 0));
+    const uint32_t srow = (uint32_t)wrow * SG;
+    if constexpr (GS == 8) {
+      b.s = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                           rs, ((srow + step0 * 2u) * 2u) | oob, 0, 0));
+    } else if constexpr (GS == 4) {
+      const uint2v v = __builtin_bit_cast(
+          uint2v, __builtin_amdgcn_raw_buffer_load_b64(rs, ((srow + step0) * 2u) | oob, 0, 0));
+      b.s[0] = v[0];
+      b.s[1] = v[1];
+    } else if constexpr (GS == 2) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        b.s[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+            rs, ((srow + ((2u * step0 + 4u * i) >> gshift)) * 2u) | oob, 0, 0);
+    }
+  };
+  auto bstore = [&](const WBatch& b) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 8 * i + wr8;
+      wl[8 * r + (wp8 ^ ((r >> 1) & 7))] = b.w[i];
+    }
+  };
+  auto wread = [&](int u) { return wl[8 * li + ((2 * u + lh) ^ ((li >> 1) & 7))]; };
+  // Scale of this lane's chunk in step u of a batch; past K (whose loads
+  // may hold the next row's scales) zero.
+  auto bscale = [&](const uint4v& sv, int t, int u) {
+    const uint32_t w = GS == 8 ? sv[u] >> (16 * lh) : GS == 4 ? sv[u >> 1] >> (16 * (u & 1)) : sv[u >> 1];
+    const bool in_k = (kg * T + t) * kTK + 32 * lh < a.K;
+    return __builtin_bit_cast(half_t, (uint16_t)(in_k ? w : 0u));
   };
   auto xstore = [&](const XStage& g, int buf, int j) {
     const half8v x = g.x[j];
@@ -666,11 +732,11 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
   // next step) stored into buffer buf ^ 1 among the MFMAs.  After the last
   // step the stage holds the zeros loaded past K; storing them into the
   // idle buffer is harmless and keeps the step one basic block.
-  auto step = [&](int buf, const WStage& ws, const XStage& xn) {
+  auto step = [&](int buf, const uint4v& ww, half_t sc, const XStage& xn) {
     const half8v* xb = lds[kg][buf];
     auto afrag = [&](int mi, int ks) { return xb[((32 * mi + li) * kTLD + 32 * lh + 8 * ks) / 8]; };
-    const half2v s1 = {ws.s, ws.s};
-    const half_t s16v = ws.s * (half_t)0.0625f;
+    const half2v s1 = {sc, sc};
+    const half_t s16v = sc * (half_t)0.0625f;
     const half2v s16 = {s16v, s16v};
     half8v af[2][MI];
 #pragma unroll
@@ -683,7 +749,7 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
         for (int mi = 0; mi < MI; ++mi) af[c ^ 1][mi] = afrag(mi, ks + 1);
       }
       half2v r[4];
-      unpack_word_x16(ws.w[ks], nib, zp, r);
+      unpack_word_x16(ww[ks], nib, zp, r);
       const half2v d0 = r[0] * s1, d1 = r[1] * s16, d2 = r[2] * s1, d3 = r[3] * s16;
       const half8v bop = half8v{d0[0], d0[1], d1[0], d1[1], d2[0], d2[1], d3[0], d3[1]};
 #pragma unroll
@@ -732,29 +798,74 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
   };
 
   XStage x0, x1;
-  WStage w0, w1;
-  xload(x0, 0);
-  wload(w0, 0);
-  xload(x1, 1);
-  wload(w1, 1);
+  if constexpr (GS) {
+    // Step t: X buffer t % 2 as below; W of step t + 1 read from LDS during
+    // step t, the next batch stored there in every fourth step (a wave's LDS
+    // accesses execute in order) and the one after it requested.
+    WBatch nxt;
+    bload(nxt, 0);
+    xload(x0, 0);
+    xload(x1, 1);
 #pragma unroll
-  for (int j = 0; j < XP; ++j) xstore(x0, 0, j);
-  xload(x0, 2);
-  if (threadIdx.x < kTKG) arrivals[threadIdx.x] = 0;
-  lds_barrier();
-  // Step t: W stage t&1, X buffer t&1; X stage (t+1)&1 stored into buffer
-  // (t+1)&1 and reloaded with step t+3; W stage t&1 reloaded with step t+2.
-  // Unrolled by two so the stages swap roles without copies.
-  for (int t0 = 0; t0 < T; t0 += 2) {
-    step(0, w0, x1);
-    wload(w0, t0 + 2);
-    xload(x1, t0 + 3);
-    step_sync();
-    if (t0 + 1 < T) {
-      step(1, w1, x0);
-      wload(w1, t0 + 3);
-      xload(x0, t0 + 4);
+    for (int j = 0; j < XP; ++j) xstore(x0, 0, j);
+    xload(x0, 2);
+    bstore(nxt);
+    uint4v scur = nxt.s;
+    bload(nxt, 4);
+    if (threadIdx.x < kTKG) arrivals[threadIdx.x] = 0;
+    lds_barrier();
+    uint4v wcur = wread(0);
+    for (int t0 = 0; t0 < T; t0 += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + u;
+        if (t >= T) break;
+        uint4v wnext, snext = scur;
+        if (u < 3) {
+          wnext = wread(u + 1);
+        } else {
+          bstore(nxt);
+          snext = nxt.s;
+          bload(nxt, t + 5);
+          wnext = wread(0);
+        }
+        if (u & 1) {
+          step(1, wcur, bscale(scur, t, u), x0);
+          xload(x0, t + 3);
+        } else {
+          step(0, wcur, bscale(scur, t, u), x1);
+          xload(x1, t + 3);
+        }
+        step_sync();
+        wcur = wnext;
+        scur = snext;
+      }
+    }
+  } else {
+    WStage w0, w1;
+    xload(x0, 0);
+    wload(w0, 0);
+    xload(x1, 1);
+    wload(w1, 1);
+#pragma unroll
+    for (int j = 0; j < XP; ++j) xstore(x0, 0, j);
+    xload(x0, 2);
+    if (threadIdx.x < kTKG) arrivals[threadIdx.x] = 0;
+    lds_barrier();
+    // Step t: W stage t&1, X buffer t&1; X stage (t+1)&1 stored into buffer
+    // (t+1)&1 and reloaded with step t+3; W stage t&1 reloaded with step t+2.
+    // Unrolled by two so the stages swap roles without copies.
+    for (int t0 = 0; t0 < T; t0 += 2) {
+      step(0, w0.w, w0.s, x1);
+      wload(w0, t0 + 2);
+      xload(x1, t0 + 3);
       step_sync();
+      if (t0 + 1 < T) {
+        step(1, w1.w, w1.s, x0);
+        wload(w1, t0 + 3);
+        xload(x0, t0 + 4);
+        step_sync();
+      }
     }
   }
 
@@ -1172,6 +1283,21 @@ __global__ __launch_bounds__(kThreads) void w8a16_kernel(W8Args a) {
   }
 }
 
+template <int KG, int WN, int MI>
+hipError_t launch_tile(const W4Args& a, int gs, int tiles, hipStream_t s) {
+  const KernelTag tag = ktag("w4a16_tile_gemm_kernel", KG, WN, MI);
+  const dim3 grid(tiles), block(64 * WN * KG);
+  if constexpr (KG * (MI * 9216 + WN * 4096) <= 160 * 1024 - 1024) {
+    switch (gs) {
+      case 8: return launch<&w4a16_tile_gemm_kernel<KG, WN, MI, 8>>(tag, grid, block, s, a);
+      case 4: return launch<&w4a16_tile_gemm_kernel<KG, WN, MI, 4>>(tag, grid, block, s, a);
+      case 2: return launch<&w4a16_tile_gemm_kernel<KG, WN, MI, 2>>(tag, grid, block, s, a);
+      default: break;
+    }
+  }
+  return launch<&w4a16_tile_gemm_kernel<KG, WN, MI, 0>>(tag, grid, block, s, a);
+}
+
 constexpr int w4a16_gemv_max_k() { return 32 * 256; }
 constexpr int w4a16_gemv_long_k() { return 32 * 512; }
 
@@ -1399,21 +1525,18 @@ hipError_t launch_w4a16(const W4Args& a, hipStream_t s) {
     W4Args t = a;
     t.group_sync = kgroups > 1 && (sync_env ? atoi(sync_env) != 0
                                             : steps >= (kRowTiles[mode] == 4 ? 16 : 32));
+    // W staged through LDS: power-of-two groups whose scales can be read
+    // in whole dwords.  128 x 64 tiles with four K-groups have no LDS left.
+    const bool staged = (a.group & (a.group - 1)) == 0 && a.K % (a.group == 32 ? 64 : 128) == 0;
+    const int gs = !staged ? 0 : a.group == 32 ? 8 : a.group == 64 ? 4 : 2;
     switch (mode) {
-      case 1: return launch<&w4a16_tile_gemm_kernel<1, 4, 4>>(ktag("w4a16_tile_gemm_kernel", 1, 4, 4),
-                                                               dim3(tiles_of(128, 128)), dim3(256), s, t);
-      case 2: return launch<&w4a16_tile_gemm_kernel<2, 4, 4>>(ktag("w4a16_tile_gemm_kernel", 2, 4, 4),
-                                                               dim3(tiles_of(128, 128)), dim3(512), s, t);
-      case 3: return launch<&w4a16_tile_gemm_kernel<2, 2, 4>>(ktag("w4a16_tile_gemm_kernel", 2, 2, 4),
-                                                               dim3(tiles_of(128, 64)), dim3(256), s, t);
-      case 4: return launch<&w4a16_tile_gemm_kernel<4, 2, 4>>(ktag("w4a16_tile_gemm_kernel", 4, 2, 4),
-                                                               dim3(tiles_of(128, 64)), dim3(512), s, t);
-      case 5: return launch<&w4a16_tile_gemm_kernel<4, 2, 2>>(ktag("w4a16_tile_gemm_kernel", 4, 2, 2),
-                                                               dim3(tiles_of(64, 64)), dim3(512), s, t);
-      case 6: return launch<&w4a16_tile_gemm_kernel<4, 2, 1>>(ktag("w4a16_tile_gemm_kernel", 4, 2, 1),
-                                                               dim3(tiles_of(32, 64)), dim3(512), s, t);
-      default: return launch<&w4a16_tile_gemm_kernel<8, 1, 1>>(ktag("w4a16_tile_gemm_kernel", 8, 1, 1),
-                                                                dim3(tiles_of(32, 32)), dim3(512), s, t);
+      case 1: return launch_tile<1, 4, 4>(t, gs, tiles_of(128, 128), s);
+      case 2: return launch_tile<2, 4, 4>(t, gs, tiles_of(128, 128), s);
+      case 3: return launch_tile<2, 2, 4>(t, gs, tiles_of(128, 64), s);
+      case 4: return launch_tile<4, 2, 4>(t, gs, tiles_of(128, 64), s);
+      case 5: return launch_tile<4, 2, 2>(t, gs, tiles_of(64, 64), s);
+      case 6: return launch_tile<4, 2, 1>(t, gs, tiles_of(32, 64), s);
+      default: return launch_tile<8, 1, 1>(t, gs, tiles_of(32, 32), s);
     }
   }
   constexpr int WM = 2, WN = NESO_GEMM_WN, BN = NESO_GEMM_BN;
