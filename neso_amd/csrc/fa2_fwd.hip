@@ -639,6 +639,114 @@ hipError_t launch_fa2_d(const Fa2Args& a, int d, bool causal, int ksplit, hipStr
 
 }  // namespace
 
+// ---- workgroup shape of the fast kernel, by cost ----
+//
+// Query waves, key groups and causal balancing of the fast kernel, with the
+// measured cost of each: one launch takes about
+//   a + (p + steps * s) per round of workgroups,
+// where steps are a workgroup's 64-key blocks per key group and s lies
+// between s1 (one workgroup on a CU) and s2 (as many as its waves and LDS
+// allow, the SIMDs shared).  The constants (us) are a least-squares fit to 884
+// shapes (1..96 slices, N = 48..8192, windows of 8..1024 keys) timed in every
+// shape of workgroup, rms 6-12%.  Taking the cheapest instead of the rule in
+// launch_fa2 where it promises 6% (causal 12%, its spread is larger) made
+// those shapes faster by a geometric mean of 9% / 14% (no mask, d = 64 /
+// 128), 23% / 20% (windows) and 15% / 19% (causal); the worst loss was 12%,
+// one causal shape, and 6% elsewhere.  E.g. B*H = 33 N = 900 d128 39.3 ->
+// 24.4 us, 84 x 452 d128 29.4 -> 21.7, causal 50 x 1000 d64 30.6 -> 20.1,
+// causal 6 x 7575 d128 132.7 -> 105, window 100 of 3000 x 20 d128 28.5 ->
+// 20.6, 40 of 8000 x 6 d64 15.9 -> 9.3.
+struct Fa2Shape {
+  int qwaves, ksplit, pair;
+};
+struct Fa2Cost {
+  float a, p, s1, s2;
+};
+enum Fa2Mask { kMaskNone = 0, kMaskWindow = 1, kMaskCausal = 2 };
+constexpr Fa2Shape kFa2Shapes[10] = {{2, 1, 0}, {2, 2, 0}, {2, 4, 0}, {4, 1, 0}, {4, 2, 0}};
+constexpr Fa2Shape kFa2CausalShapes[10] = {{2, 1, 0}, {2, 2, 0}, {2, 4, 0}, {2, 1, 1}, {2, 2, 1},
+                                           {2, 4, 1}, {4, 1, 1}, {4, 2, 1}, {4, 1, 2}, {4, 2, 2}};
+// [mask][head_dim 64, 128][shape]
+constexpr Fa2Cost kFa2Costs[3][2][10] = {
+    {{{0.00f, 4.63f, 0.56f, 1.27f}, {1.09f, 3.58f, 0.67f, 1.18f}, {0.14f, 4.73f, 1.12f, 1.50f},
+      {0.00f, 5.13f, 0.56f, 1.00f}, {0.00f, 5.43f, 0.96f, 1.50f}},
+     {{5.12f, 0.00f, 0.85f, 1.31f}, {3.73f, 2.22f, 1.09f, 1.20f}, {0.00f, 6.91f, 1.92f, 1.20f},
+      {0.00f, 6.64f, 0.82f, 1.69f}, {0.00f, 8.18f, 1.48f, 1.50f}}},
+    {{{0.78f, 4.36f, 0.61f, 2.04f}, {1.06f, 3.57f, 0.92f, 1.75f}, {0.92f, 3.37f, 1.80f, 1.50f},
+      {0.53f, 4.90f, 0.88f, 1.88f}, {0.00f, 5.45f, 1.51f, 1.50f}},
+     {{2.98f, 3.01f, 0.93f, 1.66f}, {3.25f, 3.06f, 1.16f, 1.50f}, {0.00f, 6.48f, 2.38f, 1.50f},
+      {0.00f, 7.01f, 1.15f, 2.63f}, {0.00f, 8.33f, 2.02f, 1.50f}}},
+    {{{5.03f, 0.00f, 0.60f, 1.98f}, {3.06f, 2.17f, 0.65f, 1.70f}, {0.00f, 5.20f, 1.13f, 1.50f},
+      {6.77f, 0.00f, 0.59f, 1.37f}, {1.14f, 3.26f, 0.69f, 1.16f}, {0.24f, 3.77f, 1.19f, 1.20f},
+      {0.00f, 4.16f, 0.63f, 1.07f}, {0.00f, 4.31f, 1.02f, 1.20f}, {5.90f, 0.00f, 0.55f, 1.44f},
+      {0.00f, 6.56f, 0.77f, 1.50f}},
+     {{0.00f, 5.37f, 1.04f, 1.44f}, {1.30f, 4.45f, 1.18f, 1.20f}, {0.00f, 6.94f, 1.98f, 1.50f},
+      {8.43f, 0.00f, 0.99f, 1.42f}, {6.68f, 1.31f, 1.16f, 1.20f}, {0.00f, 5.84f, 1.98f, 1.50f},
+      {0.32f, 5.70f, 1.06f, 1.84f}, {0.00f, 6.89f, 1.60f, 1.50f}, {6.95f, 0.64f, 0.91f, 2.36f},
+      {0.00f, 8.77f, 1.29f, 1.50f}}}};
+
+static float fa2_cost(const Fa2Args& a, int head_dim, Fa2Mask mask, int i, int cus) {
+  const Fa2Shape sh = mask == kMaskCausal ? kFa2CausalShapes[i] : kFa2Shapes[i];
+  const Fa2Cost c = kFa2Costs[mask][head_dim == 128][i];
+  const float n = (float)a.N, k = (float)sh.ksplit, q = 32.f * sh.qwaves;
+  // Workgroups, the longest and the mean one's steps, and passes.
+  int64_t wgs = (a.N + 32 * sh.qwaves - 1) / (32 * sh.qwaves);
+  float longest = ceilf(ceilf(n / 64.f) / k), mean = longest, passes = 1.f;
+  if (mask == kMaskWindow) {
+    const float span = fminf(n, q + (float)a.win_left + (float)a.win_right);
+    mean = fmaxf(1.f, (span / 64.f + (span < n ? 1.f : 0.5f)) / k);
+    longest = mean;
+  } else if (mask == kMaskCausal && sh.pair == 1) {
+    wgs = (wgs + 1) / 2;
+    passes = 2.f;
+    mean = fmaxf(2.f, ((n + q) / 64.f + 1.f) / k);
+    longest = mean;
+  } else if (mask == kMaskCausal && sh.pair == 2) {
+    wgs = ((a.N + 63) / 64 + 1) / 2;
+    longest = ceilf(n / 64.f / k);
+    mean = fmaxf(1.f, 0.75f * n / 64.f / k);
+  } else if (mask == kMaskCausal) {
+    mean = fmaxf(1.f, ((n + q) / 128.f + 0.5f) / k);
+  }
+  wgs *= a.batch_heads;
+  // Workgroups a CU holds: eight waves, 160 KiB of LDS.
+  const int occ = sh.qwaves == 4 ? 2 / sh.ksplit
+                  : head_dim == 128 ? (sh.ksplit == 1 ? 2 : 1)
+                                    : 4 / sh.ksplit;
+  const int64_t slots = (int64_t)cus * occ;
+  const float s_full = occ > 1 ? c.s2 : c.s1;
+  if (longest - mean < 1.01f) {  // even work: whole rounds, then what is left
+    const int64_t full = wgs / slots, rem = wgs % slots;
+    float t = c.a + (float)full * (c.p * passes + mean * s_full);
+    if (rem) {
+      const int r = (int)((rem + cus - 1) / cus);
+      const float s = occ > 1 ? c.s1 + (c.s2 - c.s1) * (float)(r - 1) / (float)(occ - 1) : c.s1;
+      t += c.p * passes + mean * s;
+    }
+    return t;
+  }
+  return c.a + c.p * passes * (float)((wgs + slots - 1) / slots) +
+         fmaxf(longest * c.s1, mean * (float)wgs / (float)slots * s_full);
+}
+
+// The shape to use instead of `now` (qwaves 0: the generic kernel).
+static Fa2Shape fa2_cheapest(const Fa2Args& a, int head_dim, Fa2Mask mask, Fa2Shape now, int cus) {
+  const int count = mask == kMaskCausal ? 10 : 5;
+  const Fa2Shape* shapes = mask == kMaskCausal ? kFa2CausalShapes : kFa2Shapes;
+  int best = -1;
+  float best_t = 0.f, now_t = -1.f;
+  for (int i = 0; i < count; ++i) {
+    const float t = fa2_cost(a, head_dim, mask, i, cus);
+    if (best < 0 || t < best_t) {
+      best = i;
+      best_t = t;
+    }
+    if (shapes[i].qwaves == now.qwaves && shapes[i].ksplit == now.ksplit && shapes[i].pair == now.pair) now_t = t;
+  }
+  if (now_t < 0.f && now.qwaves) return now;  // a shape the model does not hold
+  return now_t >= 0.f && best_t > now_t * (mask == kMaskCausal ? 0.88f : 0.94f) ? now : shapes[best];
+}
+
 int fa2_query_block() { return kBM; }  // the largest query block of any FA2 kernel
 
 hipError_t launch_fa2(Fa2Args a, int head_dim, bool causal, int bias_kind, bool out_f16,
@@ -664,7 +772,19 @@ hipError_t launch_fa2(Fa2Args a, int head_dim, bool causal, int bias_kind, bool 
   const bool bias = bias_kind != kBiasNone;
   const bool fast_ok = a.allow_fast && fa2_fast_supported(head_dim, bias_kind, in_f32) &&
                        (!bias || fabsf(a.scale_log2) >= 1e-20f);
-  if (fast_ok && (a.allow_fast == 2 || fa2_fast_preferred(causal, a.N, head_dim, small, bias))) {
+  // Without a bias and with nothing forced, the workgroup shape goes by cost.
+  // N = 128 keeps its 128-query workgroup (test_fa2_kernel_choice).
+  const bool by_cost = fast_ok && !bias && a.allow_fast == 1 && a.qwaves == 0 && a.ksplit <= 0 &&
+                       a.pair_qblocks < 0 && a.N != kBM;
+  const Fa2Mask mask = !causal ? kMaskNone : full_causal ? kMaskCausal : kMaskWindow;
+  const bool preferred = fast_ok && fa2_fast_preferred(causal, a.N, head_dim, small, bias);
+  if (by_cost && !preferred) {
+    const Fa2Shape sh = fa2_cheapest(a, head_dim, mask, Fa2Shape{0, 0, 0}, (int)cus);
+    a.qwaves = sh.qwaves;
+    a.pair_qblocks = sh.pair;
+    return launch_fa2_fast(a, head_dim, causal, bias, out_f16, sh.ksplit, stream);
+  }
+  if (fast_ok && (a.allow_fast == 2 || preferred)) {
     // Causal grids of at least two workgroups per CU: each workgroup takes a
     // long and a short query block (pair_qblocks), which evens out the work,
     // and the key split then follows the halved grid (fast kernel, measured:
@@ -702,6 +822,14 @@ hipError_t launch_fa2(Fa2Args a, int head_dim, bool causal, int bias_kind, bool 
     if (a.qwaves == 2 && a.ksplit <= 0 && a.pair_qblocks != 1) {
       const int64_t wgs64 = (int64_t)((a.N + 63) / 64) * a.batch_heads;
       ksplit = (wgs64 <= cus && a.N >= 1024) ? 4 : 2;
+    }
+    if (by_cost) {
+      // Halves need four query waves and full causal rows, pairs a mask.
+      const int pair = !causal || (a.pair_qblocks == 2 && (a.qwaves != 4 || !full_causal)) ? 0 : a.pair_qblocks;
+      const Fa2Shape sh = fa2_cheapest(a, head_dim, mask, Fa2Shape{a.qwaves, ksplit, pair}, (int)cus);
+      a.qwaves = sh.qwaves;
+      a.pair_qblocks = sh.pair;
+      ksplit = sh.ksplit;
     }
     return launch_fa2_fast(a, head_dim, causal, bias, out_f16, ksplit, stream);
   }

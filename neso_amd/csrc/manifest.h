@@ -133,7 +133,7 @@ constexpr char kManifest[] = R"JSON({
       "QW",
       "BIAS"
      ],
-     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias where measured faster than fa2_fwd_kernel (fa2_fast_preferred), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
+     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias (QW, KSPLIT, PAIR and HALVES of least measured cost, fa2_cheapest; the rules below with a bias, at N = 128, where a shape is forced, and where the cost promises too little to leave them), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -160,7 +160,7 @@ constexpr char kManifest[] = R"JSON({
       "F32IN",
       "QW"
      ],
-     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and unbiased shapes where it is measured faster; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
+     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and calls forced to it; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -295,7 +295,7 @@ constexpr char kManifest[] = R"JSON({
       "F32IN",
       "QW"
      ],
-     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and unbiased shapes where it is measured faster; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
+     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and calls forced to it; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -410,7 +410,7 @@ constexpr char kManifest[] = R"JSON({
       "QW",
       "BIAS"
      ],
-     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias where measured faster than fa2_fwd_kernel (fa2_fast_preferred), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
+     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias (QW, KSPLIT, PAIR and HALVES of least measured cost, fa2_cheapest; the rules below with a bias, at N = 128, where a shape is forced, and where the cost promises too little to leave them), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -437,7 +437,7 @@ constexpr char kManifest[] = R"JSON({
       "F32IN",
       "QW"
      ],
-     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and unbiased shapes where it is measured faster; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
+     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and calls forced to it; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -576,7 +576,7 @@ constexpr char kManifest[] = R"JSON({
       "QW",
       "BIAS"
      ],
-     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias where measured faster than fa2_fwd_kernel (fa2_fast_preferred), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
+     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias (QW, KSPLIT, PAIR and HALVES of least measured cost, fa2_cheapest; the rules below with a bias, at N = 128, where a shape is forced, and where the cost promises too little to leave them), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -603,7 +603,7 @@ constexpr char kManifest[] = R"JSON({
       "F32IN",
       "QW"
      ],
-     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and unbiased shapes where it is measured faster; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
+     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and calls forced to it; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -752,7 +752,7 @@ constexpr char kManifest[] = R"JSON({
       "QW",
       "BIAS"
      ],
-     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias where measured faster than fa2_fwd_kernel (fa2_fast_preferred), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
+     "when": "fp16 Q/K/V at head_dim 64 or 128: without a bias (QW, KSPLIT, PAIR and HALVES of least measured cost, fa2_cheapest; the rules below with a bias, at N = 128, where a shape is forced, and where the cost promises too little to leave them), and with the f32 bias table whenever |scale| >= 1e-20 (BIAS 2: the table entries of a workgroup's rows, 32 * QW + N - 1, loaded once into the band slots' LDS when they fit, KSPLIT * QW * 2 * 128 or 64 floats; BIAS 1: per-block bands otherwise); KSPLIT key groups of QW query waves (QW = 2 on grids whose 128-query workgroups fill at most half the CUs, from N = 512 without a bias, with KSPLIT = 4 while cdiv(N, 64) * batch_heads <= cus and N >= 1024, else 2); PAIR (causal grids of >= 2 workgroups per CU with QW = 4; head_dim 128 causal without a window from N = 2048 when cdiv(cdiv(N, 64), 2) * batch_heads <= cus with QW = 2, KSPLIT = 4): each workgroup takes query blocks x and nqb-1-x; HALVES (causal without a window, fewer than 2 workgroups per CU, QW = 4): each workgroup takes the 64-row blocks x and cdiv(N, 64)-1-x",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
@@ -779,7 +779,7 @@ constexpr char kManifest[] = R"JSON({
       "F32IN",
       "QW"
      ],
-     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and unbiased shapes where it is measured faster; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
+     "when": "every other FA2 call: the dense f16 bias (BIAS 2), the f32 table (BIAS 1) with |scale| < 1e-20, fp32 input (F32IN), head_dim 32, and calls forced to it; QW query waves (2 on grids that fill at most half the CUs) and KSPLIT key groups per workgroup",
      "threadgroup_size": "64 * QW * KSPLIT",
      "num_warps": "QW * KSPLIT",
      "grid": [
