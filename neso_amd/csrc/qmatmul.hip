@@ -616,7 +616,8 @@ __global__ __launch_bounds__(64 * WN * kTKG) void w4a16_tile_gemm_kernel(W4Args 
   const int ntiles = (a.N + TN - 1) / TN;
   const int id = (int)xcd_swizzle(blockIdx.x, (uint32_t)(mtiles * ntiles));
   const int m0 = (id % mtiles) * TM, n0 = (id / mtiles) * TN;
-  const int KW = a.K >> 3, SG = a.K / a.group;
+  // Staged groups are powers of two: scales per row without a division.
+  const int KW = a.K >> 3, SG = GS ? a.K >> __builtin_ctz(a.group) : a.K / a.group;
   const int mrows = __builtin_amdgcn_readfirstlane(min(TM, a.M - m0));
   const int nrows = __builtin_amdgcn_readfirstlane(min(TN, a.N - n0));
   const rsrc_t rx = make_rsrc(a.X + (int64_t)m0 * a.ldx, (uint32_t)(((int64_t)(mrows - 1) * a.ldx + a.K) * 2));

@@ -47,21 +47,25 @@ __global__ __launch_bounds__(WV * kWave) void w4a16_skinny_lds_kernel(W4Args a) 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lg = lane >> 4;
-  const int KW = a.K >> 3, SG = a.K / a.group;
+  const int gshift = __builtin_ctz(a.group >> 7);  // GS = 1: 2^gshift quads per scale
+  // Scales per row by shifts: a division here delays the first loads (1-2%
+  // of a launch).
+  const int KW = a.K >> 3, SG = GS == 4 ? a.K >> 5 : GS == 2 ? a.K >> 6 : a.K >> (7 + gshift);
   const int Q = a.K >> 7;                  // K % 128 == 0
   const int P = MP ? (Q + QPM - 1) / QPM : 1;
   const int QP = (Q + P - 1) / P, QW = (QP + WV - 1) / WV;
   const int ntiles = (a.N + 15) >> 4;
   const ZeroPoint zp = zero_point(a.zero);
   const Nibbles nib = nibble_consts();
-  const int gshift = __builtin_ctz(a.group >> 7);  // GS = 1: 2^gshift quads per scale
 
-  union Shared {
-    half8v xs[kLdsQuads * 4 * kWave];
-    float red[T][WV][4 * MT][kWave];
-  };
-  static_assert(sizeof(Shared) == sizeof(half8v) * kLdsQuads * 4 * kWave, "reduction fits X's space");
-  __shared__ Shared sh;
+  // The partial tiles have LDS of their own beside X at MT = 1 and take X's
+  // place, after a barrier, at MT = 2.
+  constexpr int kRed = T * WV * 4 * MT * kWave;
+  __shared__ half8v xs[kLdsQuads * 4 * kWave];
+  __shared__ float red_own[MT == 1 ? kRed : 1];
+  static_assert(kRed * sizeof(float) <= sizeof(xs) && sizeof(xs) + sizeof(red_own) <= 160 * 1024, "LDS");
+  float* const red = MT == 1 ? red_own : reinterpret_cast<float*>(xs);
+  auto red_at = [&](int i, int wv, int r, int ln) { return ((i * WV + wv) * (4 * MT) + r) * kWave + ln; };
 
   // X first: loads complete in issue order, so X (L2-resident) reaches LDS
   // while the weight burst is still arriving; issued after the weights, it
@@ -78,9 +82,24 @@ __global__ __launch_bounds__(WV * kWave) void w4a16_skinny_lds_kernel(W4Args a) 
   static_assert(WV * kWave == MT * kRowPieces, "MT rows per pass");
   const int xr = threadIdx.x / kRowPieces, pp = threadIdx.x % kRowPieces, ct = pp >> 2;
   const int xsw = 4 * (ct & 3) + (pp & 3);
-  half8v* const xdst = &sh.xs[ct * 64 + 16 * (pp & 3)];
+  half8v* const xdst = &xs[ct * 64 + 16 * (pp & 3)];
   half8v xv[kXPer];
+  uint32_t xslot[MP ? 1 : kXPer];
   auto xload = [&](int p) {
+    if constexpr (!MP) {
+      // One phase: per-piece offsets and slots into one buffer, which issue
+      // sooner than a buffer base per row (1-3% of a launch).
+      const rsrc_t rx = make_rsrc(a.X, (uint32_t)(((int64_t)(a.M - 1) * a.ldx + a.K) * 2));
+#pragma unroll
+      for (int i = 0; i < kXPer; ++i) {
+        const uint32_t e = threadIdx.x + i * WV * kWave;
+        const uint32_t m = e / kRowPieces, pc = e % kRowPieces, c = pc >> 2, g = pc & 3;
+        const uint32_t oob = ((int)c < 4 * Q && (int)m < a.M) ? 0u : kOut;
+        xv[i] = buf_load_half8(rx, ((m * (uint32_t)a.ldx + 8u * pc) * 2u) | oob);
+        xslot[i] = c * 64 + 16 * g + (m ^ (4 * (c & 3) + g));
+      }
+      return;
+    }
     const int cend = 4 * (min((p + 1) * QP, Q) - p * QP);  // chunks of the phase
     const uint32_t off = ((uint32_t)xr * (uint32_t)a.ldx + 8u * pp) * 2u | (ct < cend ? 0u : kOut);
 #pragma unroll
@@ -96,8 +115,8 @@ __global__ __launch_bounds__(WV * kWave) void w4a16_skinny_lds_kernel(W4Args a) 
     for (int i = 0; i < kXPer; ++i) {
       const int m = xr + MT * i;
       const half8v x = xv[i];
-      xdst[(m >> 4) * (4 * QPM * 64) + ((m & 15) ^ xsw)] =
-          half8v{x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7]};
+      half8v* const dst = MP ? xdst + (m >> 4) * (4 * QPM * 64) + ((m & 15) ^ xsw) : xs + xslot[MP ? 0 : i];
+      *dst = half8v{x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7]};
     }
   };
 
@@ -161,7 +180,7 @@ __global__ __launch_bounds__(WV * kWave) void w4a16_skinny_lds_kernel(W4Args a) 
         const half8v bv = {d0[0], d0[1], d1[0], d1[1], d2[0], d2[1], d3[0], d3[1]};
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const half8v xa = sh.xs[(mt * 4 * QPM + 4 * q + t) * kWave + 16 * lg + (li ^ (4 * t + lg))];
+          const half8v xa = xs[(mt * 4 * QPM + 4 * q + t) * kWave + 16 * lg + (li ^ (4 * t + lg))];
           acc[i][mt] = mfma16x16x32(xa, bv, acc[i][mt]);
         }
       }
@@ -172,36 +191,47 @@ __global__ __launch_bounds__(WV * kWave) void w4a16_skinny_lds_kernel(W4Args a) 
   // every tile requested up front, the wave stalls at the load instructions
   // once the CU's outstanding-request capacity is full, and X, compute and
   // the weight stream run one after another (M = 16: 12.0 -> 9.3 us).
+  auto put = [&](int i) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[red_at(i, wave, 4 * mt + r, lane)] = acc[i][mt][r];
+  };
+
   Item it[T + 1];
   xload(0);
   load_item(it[0], 0, 0);
   xstore();
   lds_barrier();
-  for (int p = 0; p < P; ++p) {
-    if (MP && p + 1 < P) xload(p + 1);
+  if constexpr (!MP) {
 #pragma unroll
     for (int i = 0; i < T; ++i) {
-      if (i + 1 < T)
-        load_item(it[i + 1], p, i + 1);
-      else if (MP)
-        load_item(it[T], p + 1, 0);
+      if (i + 1 < T) load_item(it[i + 1], 0, i + 1);
       compute(it[i], i);
+      put(i);
     }
-    if (MP && p + 1 < P) {
-      lds_barrier();
-      xstore();
-      lds_barrier();
-      it[0] = it[T];
+  } else {
+    for (int p = 0; p < P; ++p) {
+      if (p + 1 < P) xload(p + 1);
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        if (i + 1 < T)
+          load_item(it[i + 1], p, i + 1);
+        else
+          load_item(it[T], p + 1, 0);
+        compute(it[i], i);
+      }
+      if (p + 1 < P) {
+        lds_barrier();
+        xstore();
+        lds_barrier();
+        it[0] = it[T];
+      }
     }
+    if (MT > 1) lds_barrier();
+#pragma unroll
+    for (int i = 0; i < T; ++i) put(i);
   }
-
-  lds_barrier();  // the partial tiles take X's place
-#pragma unroll
-  for (int i = 0; i < T; ++i)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sh.red[i][wave][4 * mt + r][lane] = acc[i][mt][r];
   lds_barrier();
 
   // acc[i][mt] register r of lane l is D[16 mt + 4(l/16) + r][l%16] of tile i.
@@ -210,7 +240,7 @@ __global__ __launch_bounds__(WV * kWave) void w4a16_skinny_lds_kernel(W4Args a) 
     const int tile = blockIdx.x + i * gridDim.x;
     float v = 0.f;
 #pragma unroll
-    for (int wv = 0; wv < WV; ++wv) v += sh.red[i][wv][r][ln];
+    for (int wv = 0; wv < WV; ++wv) v += red[red_at(i, wv, r, ln)];
     const int m = 16 * (r >> 2) + 4 * (ln >> 4) + (r & 3);
     const int n = tile * 16 + (ln & 15);
     if (tile < ntiles && m < a.M && n < a.N) a.Y[(int64_t)m * a.ldy + n] = (half_t)v;
