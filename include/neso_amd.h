@@ -3,10 +3,11 @@
  *
  * Every entry point takes device pointers the caller owns, sizes and element
  * strides by value, and an optional HIP stream (`void*` = hipStream_t, NULL =
- * the null stream).  Nothing here allocates, copies or synchronises: a call
- * validates its arguments on the host, enqueues one kernel on `stream`
- * (neso_w8a16_matmul_ws: one or two) and returns.  Validation happens before any HIP call, so argument errors are
- * reported on hosts without a GPU.
+ * the null stream).  A call validates its arguments on the host, enqueues one
+ * kernel on `stream` (neso_w8a16_matmul_ws: one or two) and returns; it
+ * allocates, copies and synchronises nothing, except that neso_abs_max_wait
+ * waits for the kernel of its neso_abs_max_begin.  Validation happens before
+ * any HIP call, so argument errors are reported on hosts without a GPU.
  *
  * fp16 buffers are IEEE binary16, passed as `const void*`.
  *

@@ -1212,6 +1212,8 @@ bool fa2_fast_supported(int head_dim, int bias_kind, bool in_f32) {
 }
 
 bool fa2_fast_preferred(bool causal, int32_t N, int head_dim, bool small_grid, bool bias) {
+  // The rule for calls that fa2_cheapest (fa2_fwd.hip) does not decide, and
+  // the one it must beat.
   // Measured on MI355X (d = 64, B*H = 8..64): the fast kernel is ahead from
   // N = 128 up without a mask (3-15%) and for causal rows from N = 1024
   // (7-25%, growing with N); for shorter causal rows the generic kernel's

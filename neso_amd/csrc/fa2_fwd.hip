@@ -646,9 +646,11 @@ hipError_t launch_fa2_d(const Fa2Args& a, int d, bool causal, int ksplit, hipStr
 //   a + (p + steps * s) per round of workgroups,
 // where steps are a workgroup's 64-key blocks per key group and s lies
 // between s1 (one workgroup on a CU) and s2 (as many as its waves and LDS
-// allow, the SIMDs shared).  The constants (us) are a least-squares fit to 884
+// allow, the SIMDs shared).  The constants (us) are a least-squares fit to 870
 // shapes (1..96 slices, N = 48..8192, windows of 8..1024 keys) timed in every
-// shape of workgroup, rms 6-12%.  Taking the cheapest instead of the rule in
+// shape of workgroup: rms 6-10% without a mask, 9-13% with windows, 9-15%
+// causal, but 15-27% for causal pairing on 128-query workgroups and on four
+// key groups.  Taking the cheapest instead of the rule in
 // launch_fa2 where it promises 6% (causal 12%, its spread is larger) made
 // those shapes faster by a geometric mean of 9% / 14% (no mask, d = 64 /
 // 128), 23% / 20% (windows) and 15% / 19% (causal); the worst loss was 12%,

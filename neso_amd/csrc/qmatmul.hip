@@ -233,7 +233,8 @@ __global__ __launch_bounds__(kThreads) void w4a16_gemv_kernel(W4Args a) {
 }
 
 // ---------------------------------------------------------------------------
-// Skinny-M regime (3 <= M <= 64 by default): split-K MFMA.
+// Skinny-M regime: split-K MFMA, for the M <= 16 shapes that launch_w4a16
+// gives neither to the X-in-LDS kernel nor to the tile GEMM.
 //
 // A workgroup owns 16*NT rows of W (output columns n) and 16*MT rows of X.
 // Its WV waves split K into contiguous ranges of chunk quads (a quad = 4

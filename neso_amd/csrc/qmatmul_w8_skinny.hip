@@ -19,10 +19,11 @@
 //
 // int8 -> f16 is exact: 0x6400 | (b ^ 0x80) is f16 1024 + 128 + b.
 //
-// Measured per launch (rotated weights, graph of launches) against the 128 x
-// 128-tile kernel that served these calls: K 4096, N 4096 M = 1 8.5 us (2.0
-// TB/s), M = 16 9.4, M = 64 17.5, before 57 us at any M; K 4096, N 11008
-// M = 1 13.8 us (3.3 TB/s); K 11008, N 4096 M = 1 12.6 us (3.6 TB/s).  A
+// Measured per call, both launches (rotated weights, graph of launches),
+// against the 128 x 128-tile kernel that served these calls, M = 1 / 16 / 64:
+// K 4096, N 4096 44.4 / 44.5 / 45.0 -> 8.4 / 9.3 / 17.5 us (M = 1 2.0 TB/s);
+// K 4096, N 11008 48.6 / 48.7 / 49.2 -> 13.6 / 15.4 / 27.6 (3.3 TB/s);
+// K 11008, N 4096 122.6 / 122.2 / 122.8 -> 12.5 / 14.6 / 25.2 (3.6 TB/s).  A
 // kernel that only reads such strips takes 4.9, 9.1 and 9.2 us; the
 // reduction's launch is about 2.5 us of the rest.  Four or eight waves per
 // workgroup, the order of strips and splits over the XCDs, and more than two

@@ -297,7 +297,7 @@ def flash_attention_fwd(Q, K, V, O, N: int, stride_qo: int, stride_kv: int, scal
     the reference's generator (:79-89); for tensors it follows Q's dtype.
     The fp32 kernel splits each element into fp16 hi + lo; with
     ``check_range`` (default) the largest |x| of each fp32 tensor is
-    measured first (one device reduction per input and one synchronisation)
+    measured first (one kernel for all inputs, whose result the host polls)
     and a tensor outside [2^-2, 2^15) is replaced by an exact power-of-two
     rescaled copy, its factor folded into ``scale`` (Q, K) or undone on O
     (V), so any finite magnitude keeps fp32-class accuracy.  Without it, or
@@ -496,8 +496,8 @@ def rel_pos_precompute(Q, K_rel, bias_u, bias_v, T: int, d: int, nh: int, scale:
     Q, K_rel, bias_u, bias_v are contiguous fp32 [nh, T, d], [nh, 2T-1, d],
     [nh, d], [nh, d].  The bias is formed from fp16 hi + lo splits of
     Q + bias_v and K_rel, so their elements must lie below 65504 in
-    magnitude; ``check_range`` verifies that before the launch (device
-    reductions and a synchronisation, skipped under graph capture).
+    magnitude; ``check_range`` verifies that before the call returns (one
+    kernel whose result the host polls, skipped under graph capture).
     """
     _rel_pos_precompute(Q, K_rel, bias_u, bias_v, T, d, nh, scale, Q_u, rel_bias, check_range, stream,
                         False)
